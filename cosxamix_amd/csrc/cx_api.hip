@@ -510,11 +510,55 @@ extern "C" int cx_softmax(float* x, size_t len, size_t width, void* stream) {
   return cx_launch_softmax(x, len, width, STREAM(stream));
 }
 
+// the scores of one slab of query tokens in cx_attention; the largest calls take
+// a few slabs (a slab of 64 tokens at least: 131 MB at 32 heads and 16000
+// positions)
+static const size_t kAttnSlabBytes = 256ull << 20;
+
 extern "C" int cx_attention(const float* q, const float* k, const float* v, size_t tokens,
                             size_t total, size_t heads, size_t kv_heads, size_t hd, float* out,
                             void* stream) {
   CX_REQUIRE(q && k && v && out, "attention: null pointer");
-  return cx_launch_attention(q, k, v, tokens, total, heads, kv_heads, hd, out, STREAM(stream));
+  hipStream_t s = STREAM(stream);
+  // Many query tokens on the kernels made for them, in slabs of tokens whose
+  // scores fit kAttnSlabBytes of the thread's scratch. A captured call keeps to
+  // the general kernel, which needs no scratch: a graph must not hold a
+  // buffer that a later call may replace.
+  const bool many = kv_heads && heads >= kv_heads && heads % kv_heads == 0 && tokens > 0 &&
+                    tokens <= total && total <= CX_ATT_MAX_TOTAL && heads <= 128 &&
+                    cx_attn_many_suits_general(tokens, total, heads, hd) &&
+                    (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0 && !capturing(s);
+  if (!many) return cx_launch_attention(q, k, v, tokens, total, heads, kv_heads, hd, out, s);
+  const cx_attn_many_floats s64 = cx_attn_many_scratch(64, total, heads, kv_heads);
+  auto up = [](size_t floats) { return (floats * 4 + 255) / 256 * 256; };
+  // 64 tokens are whole tiles of rows whatever the heads per group
+  size_t slab = kAttnSlabBytes / ((s64.sc + s64.cm + s64.inv) * 4) * 64;
+  slab = tokens < slab ? tokens : slab < 64 ? 64 : slab;
+  const cx_attn_many_floats f = cx_attn_many_scratch(slab, total, heads, kv_heads);
+  void* sp = nullptr;
+  cx_scratch scr(s);
+  int rc = scr.get(up(f.sc) + up(f.cm) + up(f.inv), &sp);
+  if (rc) {  // no room for the scores: the general kernel needs none
+    (void)hipGetLastError();
+    return cx_launch_attention(q, k, v, tokens, total, heads, kv_heads, hd, out, s);
+  }
+  cx_attn_many_args a{};
+  a.sc = (float*)sp;
+  a.cm = (float*)((uint8_t*)sp + up(f.sc));
+  a.inv = (float*)((uint8_t*)sp + up(f.sc) + up(f.cm));
+  a.k = k;
+  a.v = v;
+  a.heads = (uint32_t)heads;
+  a.kvh = (uint32_t)kv_heads;
+  a.hd = (uint32_t)hd;
+  for (size_t t0 = 0; t0 < tokens; t0 += slab) {
+    a.tokens = (uint32_t)(tokens - t0 < slab ? tokens - t0 : slab);
+    a.pos = (uint32_t)(total - tokens + t0);
+    a.q = q + t0 * heads * hd;
+    a.out = out + t0 * heads * hd;
+    if ((rc = cx_launch_attn_many(a, s))) return rc;
+  }
+  return CX_OK;
 }
 
 extern "C" int cx_attention_decode(const float* q, const float* k, const float* v, size_t total,
@@ -679,7 +723,7 @@ struct cx_model {
 struct cx_prefill {
   uint32_t T;
   float *x, *nrm, *q, *k, *v, *att, *g, *u, *tmp;  // nrm also holds the SwiGLU rows
-  float *sc, *cm;
+  float *sc, *cm, *inv;
   void* scratch;
 };
 
@@ -1281,7 +1325,7 @@ extern "C" void cx_cache_free(cx_cache* c) {
   void* bufs[] = {c->kv,   c->hist, c->st,   c->pm,    c->pl,    c->po,  c->sc,    c->cm,
                   c->sd,   c->spb,  c->spart, c->sordp, c->sord,  P.x,    P.nrm,    P.q,
                   P.k,     P.v,     P.att,   P.g,      P.u,      P.tmp,  P.sc,     P.cm,
-                  P.scratch};
+                  P.inv,    P.scratch};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   if (c->htok) (void)hipHostFree(c->htok);
@@ -1511,49 +1555,62 @@ static int run_steps(cx_cache* C, size_t prompt_end, size_t steps, float* step_m
 // Modelo::forward over several tokens (src/forward.rs:375-505) as one pass
 // per layer over a chunk of up to T tokens. The GEMVs become the int8 MFMA
 // contraction for Q4_K/Q5_K (other types run the GEMV row by row), and the
-// attention runs the decode step's kernels with one query token per grid
-// slice. Every value equals what token-by-token decoding computes:
+// attention takes the chunk's tokens at once. Every value equals what token-by-token decoding computes:
 // - the contraction is bit-identical to the GEMV;
 // - the rows are normalized in the fused GEMV prologue's tree;
 // - the quantization of a row is a function of its values alone;
 // - bias and residual adds are the same single f32 adds as the epilogues;
-// - the attention kernels and their path (exact or split-K, by capacity)
-//   are the decode step's.
+// - the attention forms every score, softmax and output in the one-token
+//   kernels' order (cx_attn_many.hip for a full chunk, else the decode step's
+//   kernels with several query tokens).
 // So a prompt gives the same logits, cache and tokens either way.
-static const size_t kPrefillMaxT = 256;
-static const size_t kPrefillAttnBytes = 256ull << 20;  // attention scratch bound
+// Tokens a chunk. 512 rather than 256: the attention of many tokens spreads its
+// outputs (tokens x heads x head_dim) over the chip, and the contraction's tiles
+// fill more CUs.
+static const size_t kPrefillMaxT = 512;
+static const size_t kPrefillAttnBytes = 640ull << 20;  // attention scratch bound: 512 tokens at
+                                                       // 32 heads up to 10000 positions
 
-static int prefill_alloc(cx_cache* C) {
+static int prefill_alloc_chunk(cx_cache* C, size_t max_t, size_t attn_bytes) {
   cx_prefill& P = C->pf;
-  if (P.T) return CX_OK;
   const cx_config& c = C->m->cfg;
   const size_t D = c.dim, hd = D / c.heads, kvd = c.kv_heads * hd, I = c.ffn, H = c.heads;
   const size_t per_tok = (cx_attn_score_floats(H, C->cap) + cx_attn_chunk_floats(H, C->cap)) * 4;
-  size_t T = kPrefillAttnBytes / per_tok;
-  T = T > kPrefillMaxT ? kPrefillMaxT : T < 16 ? 16 : T / 16 * 16;
+  size_t T = attn_bytes / per_tok;
+  T = T > max_t ? max_t : T < 16 ? 16 : T / 16 * 16;
   if (T > C->cap) T = C->cap;
   const size_t wide = D > I ? D : I;
+  // the scratch of either attention (few and many query tokens)
+  const cx_attn_many_floats f = cx_attn_many_scratch(T, C->cap, H, c.kv_heads);
+  const size_t sc = T * cx_attn_score_floats(H, C->cap), cm = T * cx_attn_chunk_floats(H, C->cap);
   struct Want {
     float** p;
     size_t floats;
-  } want[] = {{&P.x, T * D},   {&P.nrm, T * wide}, {&P.q, T * D},   {&P.k, T * kvd},
-              {&P.v, T * kvd}, {&P.att, T * D},    {&P.g, T * I},   {&P.u, T * I},
-              {&P.tmp, T * D}};
+  } want[] = {{&P.x, T * D},   {&P.nrm, T * wide}, {&P.q, T * D}, {&P.k, T * kvd},
+              {&P.v, T * kvd}, {&P.att, T * D},    {&P.g, T * I}, {&P.u, T * I},
+              {&P.tmp, T * D}, {&P.sc, f.sc > sc ? f.sc : sc},    {&P.cm, f.cm > cm ? f.cm : cm},
+              {&P.inv, f.inv}};
+  bool ok = true;
+  for (const Want& w : want) ok = ok && hipMalloc(w.p, w.floats * 4) == hipSuccess;
+  ok = ok && hipMalloc(&P.scratch, cx_gemm_scratch_bytes(T, wide)) == hipSuccess;
+  if (ok) {
+    P.T = (uint32_t)T;
+    return CX_OK;
+  }
   for (const Want& w : want)
-    if (hipMalloc(w.p, w.floats * 4) != hipSuccess) goto fail;
-  if (hipMalloc(&P.sc, T * cx_attn_score_floats(H, C->cap) * 4) != hipSuccess ||
-      hipMalloc(&P.cm, T * cx_attn_chunk_floats(H, C->cap) * 4) != hipSuccess)
-    goto fail;
-  if (hipMalloc(&P.scratch, cx_gemm_scratch_bytes(T, wide)) != hipSuccess) goto fail;
-  P.T = (uint32_t)T;
-  return CX_OK;
-fail:
-  for (void* b : {(void*)P.x, (void*)P.nrm, (void*)P.q, (void*)P.k, (void*)P.v, (void*)P.att,
-                  (void*)P.g, (void*)P.u, (void*)P.tmp, (void*)P.sc, (void*)P.cm, P.scratch})
-    if (b) (void)hipFree(b);
+    if (*w.p) (void)hipFree(*w.p);
+  if (P.scratch) (void)hipFree(P.scratch);
   P = cx_prefill{};
+  (void)hipGetLastError();
   cx_set_error("prefill: cannot allocate the buffers of %zu tokens", T);
   return CX_ENOMEM;
+}
+
+// the buffers at the cache's first prefill; shorter chunks where memory is short
+static int prefill_alloc(cx_cache* C) {
+  if (C->pf.T) return CX_OK;
+  const int rc = prefill_alloc_chunk(C, kPrefillMaxT, kPrefillAttnBytes);
+  return rc ? prefill_alloc_chunk(C, kPrefillMaxT / 2, kPrefillAttnBytes / 4) : rc;
 }
 
 // out[r] = W . in[r] for `rows` rows of width k: the MFMA contraction,
@@ -1631,8 +1688,8 @@ static int prefill_linear(cx_cache* C, const int* type, const uint8_t* const* w,
   return CX_OK;
 }
 
-// tokens at positions [st->pos, st->pos + nt), already in hist: the layers
-static int enqueue_prefill_chunk(cx_cache* C, uint32_t nt) {
+// tokens at positions [pos, pos + nt) (pos = st->pos), already in hist: the layers
+static int enqueue_prefill_chunk(cx_cache* C, uint32_t pos, uint32_t nt) {
   cx_model* m = C->m;
   cx_prefill& P = C->pf;
   const cx_config& c = m->cfg;
@@ -1659,20 +1716,38 @@ static int enqueue_prefill_chunk(cx_cache* C, uint32_t nt) {
     if ((rc = cx_launch_rope_kv(P.q, P.k, P.v, kc, vc, m->cos_t, m->sin_t, c.heads, c.kv_heads,
                                 hd, C->st, nt, s)))
       return rc;
-    cx_attn_args a{};
-    a.q = P.q;
-    a.kc = kc;
-    a.vc = vc;
-    a.heads = c.heads;
-    a.kvh = c.kv_heads;
-    a.hd = hd;
-    a.cap = (uint32_t)C->cap;
-    a.st = C->st;
-    a.sc = P.sc;
-    a.cm = P.cm;
-    a.out = P.att;
-    a.tokens = nt;
-    if ((rc = cx_launch_attn_decode(a, s))) return rc;
+    if (cx_attn_many_suits_prefill(nt, pos + nt, c.heads, hd)) {
+      cx_attn_many_args a{};
+      a.q = P.q;
+      a.k = kc;
+      a.v = vc;
+      a.tokens = nt;
+      a.pos = pos;
+      a.heads = c.heads;
+      a.kvh = c.kv_heads;
+      a.hd = hd;
+      a.sc = P.sc;
+      a.cm = P.cm;
+      a.inv = P.inv;
+      a.out = P.att;
+      rc = cx_launch_attn_many(a, s);
+    } else {
+      cx_attn_args a{};
+      a.q = P.q;
+      a.kc = kc;
+      a.vc = vc;
+      a.heads = c.heads;
+      a.kvh = c.kv_heads;
+      a.hd = hd;
+      a.cap = (uint32_t)C->cap;
+      a.st = C->st;
+      a.sc = P.sc;
+      a.cm = P.cm;
+      a.out = P.att;
+      a.tokens = nt;
+      rc = cx_launch_attn_decode(a, s);
+    }
+    if (rc) return rc;
     // src/forward.rs:466-491
     qd = 0;
     {  // x += att . o^T
@@ -1723,7 +1798,7 @@ static int prefill(cx_cache* C, size_t t) {
   for (size_t c0 = 0; c0 < t; c0 += P.T) {
     const uint32_t nt = (uint32_t)(t - c0 < P.T ? t - c0 : P.T);
     if ((rc = cx_launch_set_state(C->st, (uint32_t)(C->len + c0), end, cap, s)) ||
-        (rc = enqueue_prefill_chunk(C, nt)))
+        (rc = enqueue_prefill_chunk(C, (uint32_t)(C->len + c0), nt)))
       return rc;
     last = nt - 1;
   }

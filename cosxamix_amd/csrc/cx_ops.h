@@ -94,6 +94,26 @@ int cx_launch_attn_exact(const cx_attn_args& a, float scale, hipStream_t s);
 // cm[h][chunk] of every head, any cache length (rope and the KV append
 // as k_attn_scores)
 int cx_launch_att_scores(const cx_attn_args& a, float scale, hipStream_t s);
+// Many query tokens (cx_attn_many.hip): token z at position pos + z against
+// the cached positions 0 .. pos + z of k and v ([..][kvh*hd], already holding
+// them), q and out rows of heads*hd; sc, cm and inv are scratch of at least
+// cx_attn_many_scratch(tokens, pos + tokens, heads, kvh) floats. Order-exact.
+struct cx_attn_many_args {
+  const float *q, *k, *v;  // 16-byte aligned
+  uint32_t tokens, pos, heads, kvh, hd;
+  float *sc, *cm, *inv;
+  float* out;
+};
+struct cx_attn_many_floats {
+  size_t sc, cm, inv;
+};
+// whether `tokens` query tokens (the last of `total` positions) are better
+// served by cx_launch_attn_many than by cx_launch_attn_decode, and than by
+// cx_launch_attention
+bool cx_attn_many_suits_prefill(size_t tokens, size_t total, size_t heads, size_t hd);
+bool cx_attn_many_suits_general(size_t tokens, size_t total, size_t heads, size_t hd);
+cx_attn_many_floats cx_attn_many_scratch(size_t tokens, size_t total, size_t heads, size_t kvh);
+int cx_launch_attn_many(const cx_attn_many_args& a, hipStream_t s);
 int cx_launch_attention(const float* q, const float* k, const float* v, size_t tokens,
                         size_t total, size_t heads, size_t kvh, size_t hd, float* out,
                         hipStream_t s);

@@ -1,0 +1,96 @@
+"""Attention of many query tokens (cx_attn_many.hip) through ops.atencion, bit
+for bit against the oracle's ops::atencion (src/ops.rs:1258-1325), at the edges of
+its tiles: rows (tokens x heads per group) around 64 and 128, positions around 32,
+64 and 128, one to sixteen heads per group, both head dims, and every row count a
+lane takes. Values that a row does not see may be anything; a captured call and
+misaligned rows take the general kernel."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def inputs(seed, tokens, total, heads, kv, hd):
+    r = np.random.default_rng(seed)
+    return (r.normal(0, 1, (tokens, heads * hd)).astype(np.float32),
+            r.normal(0, 1, (total, kv * hd)).astype(np.float32),
+            r.normal(0, 1, (total, kv * hd)).astype(np.float32))
+
+
+def run(dev, q, k, v, heads, kv, hd):
+    from cosxamix_amd import ops
+    out = torch.full(q.shape, 7.0, dtype=torch.float32, device=dev)
+    ops.atencion(torch.from_numpy(q).to(dev), torch.from_numpy(k).to(dev),
+                 torch.from_numpy(v).to(dev), (len(q), len(k), heads, kv, hd), out)
+    return out.cpu().numpy()
+
+
+def same(got, want):  # equal bits; a NaN equals a NaN
+    got, want = got.reshape(-1), np.asarray(want, np.float32).reshape(-1)
+    return np.all((got.view(np.uint32) == want.view(np.uint32)) |
+                  (np.isnan(got) & np.isnan(want)))
+
+
+def oracle(q, k, v, heads, kv, hd):
+    return O.attention(q.reshape(-1), k.reshape(-1), v.reshape(-1), len(q), len(k), heads, kv, hd)
+
+
+@pytest.mark.parametrize("tokens,total,heads,kv,hd", [
+    (1, 1024, 4, 4, 64), (2, 1025, 3, 1, 128), (63, 1151, 2, 2, 64), (64, 1024, 1, 1, 128),
+    (65, 1153, 7, 1, 64), (8, 1087, 16, 2, 128), (9, 1089, 32, 2, 64), (300, 300, 14, 2, 64),
+    (257, 511, 16, 2, 128), (129, 1500, 8, 8, 128), (1100, 1100, 4, 1, 64)])
+def test_many_tokens_bit_exact(dev, tokens, total, heads, kv, hd):
+    q, k, v = inputs(tokens * 7 + total, tokens, total, heads, kv, hd)
+    assert same(run(dev, q, k, v, heads, kv, hd), oracle(q, k, v, heads, kv, hd))
+
+
+def test_large_tiles_bit_exact(dev):
+    # 128 x 128 score tiles and four rows a lane: the first and last tokens
+    # against the oracle (each is the last token of its own prefix)
+    tokens, total, heads, kv, hd = 512, 1030, 32, 8, 128
+    q, k, v = inputs(5, tokens, total, heads, kv, hd)
+    got = run(dev, q, k, v, heads, kv, hd)
+    for t in (0, 1, 31, 32, 300, 510, 511):
+        n = total - tokens + t + 1
+        assert same(got[t], oracle(q[t:t + 1], k[:n], v[:n], heads, kv, hd)), t
+
+
+@pytest.mark.parametrize("tokens", [40, 300])
+def test_special_values(dev, tokens):
+    # inf and NaN where rows do not see them, a NaN key, an infinite query
+    # (its maximum is not finite), equal keys, scores down to exp's underflow
+    total, heads, kv, hd = 1100, 4, 2, 64
+    q, k, v = inputs(11, tokens, total, heads, kv, hd)
+    v[total - 1, 3] = np.inf
+    v[total - 2, 5] = np.nan
+    v[total - 5, 7] = -np.inf
+    k[total - 3] = np.nan
+    q[1] = np.inf
+    q[2] *= 60.0
+    k[100:164] = k[100]
+    assert same(run(dev, q, k, v, heads, kv, hd), oracle(q, k, v, heads, kv, hd))
+
+
+def test_capture_and_misaligned_rows_take_the_general_kernel(dev):
+    from cosxamix_amd import ops
+    tokens, total, heads, kv, hd = 70, 1040, 4, 2, 64
+    q, k, v = inputs(3, tokens, total, heads, kv, hd)
+    want = oracle(q, k, v, heads, kv, hd)
+    qd, kd, vd = (torch.from_numpy(t).to(dev) for t in (q, k, v))
+    out = torch.zeros_like(qd)
+    forma = (tokens, total, heads, kv, hd)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ops.atencion(qd, kd, vd, forma, out)
+    for _ in range(3):
+        out.fill_(7.0)
+        g.replay()
+        assert same(out.cpu().numpy(), want)
+    flat = torch.empty(q.size + 1, device=dev)
+    flat[1:] = qd.reshape(-1)
+    out.fill_(7.0)
+    ops.atencion(flat[1:].reshape(q.shape), kd, vd, forma, out)  # 4-byte aligned
+    assert same(out.cpu().numpy(), want)
