@@ -200,6 +200,18 @@ __device__ inline void cx_dma16_async(const void* g, void* l) {
       : "memory");
 }
 
+// The same from a wave-uniform base plus a byte offset a lane
+__device__ inline void cx_dma16_async_s(const void* base, uint32_t off, void* l) {
+  const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(cx_lds_ptr)l);
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
+      "global_load_lds_dwordx4 %2, %3\n\ts_nop 0\n\ts_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "s"(la), "v"(off), "s"(base)
+      : "memory");
+}
+
 // The same for 4 bytes a lane: LDS `l` + 4 * lane.
 __device__ inline void cx_dma4_async(const void* g, void* l) {
   const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(cx_lds_ptr)l);

@@ -15,9 +15,9 @@
 // within 1e-4 of the maximum (src/ops.rs:1518-1561); keeping the per-row
 // order makes a batched prefill bit-identical to token-by-token.
 //
-// The per-sub-block f32 term (6 VALU operations per output and sub-block)
-// bounds this path, not the MFMA: a 16x16x32 MFMA is followed by 24 VALU
-// instructions per lane.
+// The per-sub-block f32 term (6 VALU operations per output and sub-block in
+// k_gemm, 5 in k_gemm_w) bounds this path, not the MFMA: a 16x16x32 MFMA is
+// followed by 24 or 20 VALU instructions per lane.
 //
 // MFMA lane layout (checked on the device): A 16x32 — lane l holds row
 // l%16, k = 8(l/16)..+8 as 8 bytes; B 32x16 — lane l holds column l%16,
@@ -27,7 +27,7 @@
 // and 6-bit scales itself, from one 16-byte read of the block header, and
 // reads xe, xs of its four activation rows as float4s.
 //
-// Workgroup: 4 or 8 waves over a TW x MT tile (TW = 16 RW weight rows, MT =
+// k_gemm's workgroup: 4 or 8 waves over a TW x MT tile (TW = 16 RW weight rows, MT =
 // 16 AW WA activation rows); the waves split rows (RW), activation tiles (AW)
 // and, when a tile is too small to give every wave its own rows, the eight
 // sub-blocks of each super-block (KS). With KS > 1 the waves write their
@@ -94,6 +94,11 @@ __device__ inline void scale_min(uint32_t y, uint32_t z, uint32_t w, int j, uint
     mn = ((w >> (s + 4)) & 0xF) | (((z >> (s + 6)) & 3) << 4);
   }
 }
+
+template <bool B>
+struct Bool {
+  static constexpr bool value = B;
+};
 
 struct GemmParams {
   const uint8_t* w;     // n rows x row_bytes, GGUF raw
@@ -366,6 +371,272 @@ __global__ __launch_bounds__(64 * RW * AW * KS) void k_gemm(GemmParams P) {
         }
     }
   }
+}
+
+// ------------------------------------------------ Q4_K/Q5_K, many rows
+// The same products and terms with the weights in registers. A workgroup of 4
+// waves takes 64 weight rows x 16 WA activation rows, wave w the 16 rows from
+// 16 w: no two waves share a weight byte, so each lane loads its share straight
+// into registers, a super-block ahead; only the activation rows and their xe, xs
+// pass through LDS for the workgroup (double-buffered direct-to-LDS loads, one
+// super-block a stage, one barrier).
+//
+// Lane layout as k_gemm: lane l holds weight row l % 16 and the results of
+// activation rows 4 (l / 16) .. + 4 of each tile. The four lanes of a row decode
+// two sub-blocks' scales each, once a super-block, and pass them around by
+// ds_bpermute (two reads a sub-block): every lane decoding all eight cost ~12
+// operations a sub-block, half of them (bit-field extract, convert) at half rate.
+//
+// In LDS an activation row is its 256 bytes in 16-byte chunks, chunk c at c ^
+// (row % 16): the 16 rows that a read takes at once fall on all banks.
+//
+// E as f32 costs no conversion: the MFMA starts from the bits of E_BASE = 1.5 *
+// 2^23, so its result read as f32 is E_BASE + E exactly (|E| < 2^22), and
+// fma(ds, E_BASE + E, -ds * E_BASE) is ds * E rounded once, the reference's
+// product: ds = d * sc has at most 17 significant bits, so -ds * E_BASE is exact.
+// Where a d of the wave is not finite the product is formed the plain way. (A
+// zero may come out with the other sign; it is added to a sum that starts at
+// +0.0, which no zero changes.)
+//
+// The VALU bounds it: 5 operations an output and sub-block at ~2.5 clocks, of which
+// the four at a time that one wave can have ready run at ~3.1 with three waves a
+// SIMD. 11008 x 2048, m = 512: 84 -> 79 us (k_gemm 64 x 64), 32.8 waves' worth of
+// terms at that rate are 60; the rest is the last round of workgroups (1.8 a CU).
+// Measured beside it and dropped: weights as the A operand with the scales in an
+// LDS table (no better), 12 and 16 waves a workgroup (slower: the barrier), scales
+// by DPP or in SGPRs (conversions and scalar loads cost what they save).
+constexpr float E_BASE = 12582912.0f;
+constexpr int E_BASE_BITS = 0x4B400000;
+
+// one lane's share of a super-block of its weight row: the header, the nibbles
+// of its k group in the four sub-block pairs, and (Q5_K) its fifth bits
+template <int T> struct WRegs {
+  uint4 hd;
+  uint2 q[4], h;
+  __device__ void load(const uint8_t* blk, int G) {
+    hd = *reinterpret_cast<const uint4*>(blk);
+    if constexpr (T == CX_Q5_K) h = *reinterpret_cast<const uint2*>(blk + 16 + 8 * G);
+#pragma unroll
+    for (int p = 0; p < 4; p++)
+      q[p] = *reinterpret_cast<const uint2*>(blk + GQ<T>::BPB - 128 + 32 * p + 8 * G);
+  }
+  // every word has arrived here (the compiler's waits for them go before this)
+  __device__ void arrived() {
+    asm volatile("" : "+v"(hd.x), "+v"(hd.y), "+v"(hd.z), "+v"(hd.w));
+    pin();
+  }
+  __device__ void pin() {
+    asm volatile("" : "+v"(q[0].x), "+v"(q[0].y), "+v"(q[1].x), "+v"(q[1].y), "+v"(q[2].x),
+                 "+v"(q[2].y), "+v"(q[3].x), "+v"(q[3].y));
+    if constexpr (T == CX_Q5_K) asm volatile("" : "+v"(h.x), "+v"(h.y));
+  }
+  __device__ long operand(int j) const {
+    uint32_t lo = (q[j >> 1].x >> (4 * (j & 1))) & 0x0F0F0F0Fu;
+    uint32_t hi = (q[j >> 1].y >> (4 * (j & 1))) & 0x0F0F0F0Fu;
+    if constexpr (T == CX_Q5_K) {
+      lo |= ((h.x >> j) & 0x01010101u) << 4;
+      hi |= ((h.y >> j) & 0x01010101u) << 4;
+    }
+    return (long)(((uint64_t)hi << 32) | lo);
+  }
+};
+
+template <int NW, int WA> struct WShape {
+  static constexpr int TW = 16 * NW, MT = 16 * WA;
+  static constexpr int LX = 4 * WA, LE = WA;     // 1 KiB loads a stage: activation rows; xe, xs
+  static constexpr int STAGE = (LX + LE) * 1024;  // bytes
+  static constexpr size_t lds = 2 * STAGE;
+};
+
+template <int T, int NW, int WA, int OCC>
+__global__ __launch_bounds__(64 * NW, OCC) void k_gemm_w(GemmParams P) {
+  static_assert(NW % 4 == 0, "a wave's loads are rows of one remainder mod 16");
+  using SH = WShape<NW, WA>;
+  constexpr int TW = SH::TW, MT = SH::MT, LX = SH::LX, LE = SH::LE;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane % 16, G = lane / 16;
+  // blockIdx -> (row tile, activation tile), as k_gemm
+  const uint32_t b = blockIdx.x, A = P.act_tiles;
+  const uint32_t rt = b / (8 * A) * 8 + b % 8, at = b / 8 % A;
+  if (rt >= P.row_tiles) return;  // whole workgroup, before any load or barrier
+  const uint32_t a0 = at * MT;
+  const uint8_t* W = P.w;
+  float* DST = P.dst;
+  const float* BIAS = P.sbias[0];
+  uint32_t N = P.n, r0 = rt * TW;
+  // (constant indices: a struct argument indexed by a variable goes to scratch)
+#pragma unroll
+  for (uint32_t i = 0; i < CX_GEMM_SEGS; i++)
+    if (i < P.nseg && rt * TW >= P.sr[i]) {
+      W = P.sw[i];
+      DST = P.sd[i];
+      BIAS = P.sbias[i];
+      N = P.sr[i + 1] - P.sr[i];
+      r0 = rt * TW - P.sr[i];
+    }
+  r0 += 16 * wave;  // the wave's first row
+  const uint32_t wr = r0 + col;  // this lane's weight row (past the end: a valid row)
+  const uint8_t* wrow = W + (size_t)(wr < N ? wr : N - 1) * P.row_bytes;
+  // Load l of a stage (l = wave, wave + NW, ...) fills its chunks 64 l + lane: for
+  // l < LX the activation rows 4 l .. + 4 (a wave's l agree mod 4, so the lanes'
+  // offsets are the same in each and the row a uniform base), then xe and xs, of
+  // which a wave has one load at most.
+  const uint32_t xoff = (lane / 16) * P.k + 16 * ((lane % 16) ^ ((4 * wave + lane / 16) % 16));
+  const uint32_t el = (wave + NW - LX % NW) % NW, ec = 64 * el + lane;
+  const uint32_t eoff =  // sub-block ec / (MT / 2): MT xe, then MT xs
+      (2 * (ec / (MT / 2)) + ec % (MT / 2) / (MT / 4)) * P.m_pad * 4 + 16 * (ec % (MT / 4));
+  const int8_t* xbase = P.xq + (size_t)a0 * P.k;
+  const float* ebase = P.xexs + a0;
+  auto issue = [&](uint32_t sb) {
+    uint8_t* l = lds + (sb & 1) * SH::STAGE;
+#pragma unroll
+    for (int u = 0; u < (LX + NW - 1) / NW; u++) {
+      const int i = wave + NW * u;
+      if (i < LX) cx_dma16_async_s(xbase + (size_t)(4 * i) * P.k + 256 * sb, xoff, l + 1024 * i);
+    }
+    if (el < (uint32_t)LE)
+      cx_dma16_async_s(ebase + (size_t)sb * 16 * P.m_pad, eoff, l + 1024 * (LX + el));
+  };
+  float acc[WA][4];
+#pragma unroll
+  for (int t = 0; t < WA; t++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[t][i] = 0.0f;
+  const uint32_t nb = P.nb;
+  WRegs<T> wn;
+  wn.load(wrow, G);
+  issue(0);
+#pragma unroll 1
+  for (uint32_t sb = 0; sb < nb; sb++) {
+    cx_wait_vm<0>();  // this wave's part of stage sb, and its weights
+    cx_wait_lds();
+    cx_barrier();     // every wave's part; stage sb - 1 is read
+    WRegs<T> w = wn;
+    // before the next loads are issued: a wait that the compiler placed later
+    // would count the direct-to-LDS loads, which it does not know of, as done
+    w.arrived();
+    if (sb + 1 < nb) issue(sb + 1);
+    wn.load(wrow + (size_t)(sb + 1 < nb ? sb + 1 : sb) * GQ<T>::BPB, G);
+    const uint8_t* X = lds + (sb & 1) * SH::STAGE;
+    const float* E = reinterpret_cast<const float*>(X + 256 * MT) + 4 * G;
+    // sub-blocks 2G and 2G + 1 of this lane's row: for G < 2 the 6-bit fields
+    // themselves, else 4 bits of the third scale word and 2 of the others
+    const bool wild = __any((w.hd.x & 0x7C00u) == 0x7C00u);
+    float ds2[2], dm2[2];
+    {
+      const float d = cx_h2f(w.hd.x & 0xFFFFu), dmin = cx_h2f(w.hd.x >> 16);
+      const uint32_t sh = 16 * (G & 1);
+      const uint32_t y = w.hd.y >> sh, z = w.hd.z >> sh, v = w.hd.w >> sh;
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const uint32_t yb = (y >> (8 * u)) & 0xFFu, zb = (z >> (8 * u)) & 0xFFu,
+                       vb = (v >> (8 * u)) & 0xFFu;
+        const uint32_t sc = G < 2 ? yb & 63u : (vb & 15u) | ((yb >> 6) << 4);
+        const uint32_t mn = G < 2 ? zb & 63u : (vb >> 4) | ((zb >> 6) << 4);
+        ds2[u] = d * (float)sc;
+        dm2[u] = dmin * (float)mn;
+      }
+    }
+    auto block = [&](auto fin) {
+      constexpr bool FIN = decltype(fin)::value;
+      // the activation operand: row 16 t + col, chunk (2 j + G / 2) ^ col. (ax is
+      // made opaque so that the eight addresses are formed where they are used,
+      // one operation each, and not kept in eight registers.)
+      uint32_t ax = 256 * col + 16 * ((G / 2) ^ col) + 8 * (G & 1);
+      asm volatile("" : "+v"(ax));
+      auto act = [&](int j, int t) {
+        return *reinterpret_cast<const long*>(X + (ax ^ (32 * j)) + 4096 * t);
+      };
+      auto from = [&](int j, const float (&v)[2]) {  // this row's value for sub-block j
+        return __int_as_float(
+            __builtin_amdgcn_ds_bpermute(4 * col + 64 * (j / 2), __float_as_int(v[j & 1])));
+      };
+      v4i base;
+#pragma unroll
+      for (int i = 0; i < 4; i++) base[i] = FIN ? E_BASE_BITS : 0;
+      v4i e[WA];
+      float dsj[2], dmj[2];
+      dsj[0] = from(0, ds2);
+      dmj[0] = from(0, dm2);
+      // xe, xs of a tile's four activation rows, the next tile's read under this
+      // one's terms
+      float4 xeb[2], xsb[2];
+      auto scales = [&](int j, int t, int buf) {
+        const float* p = E + 2 * MT * j + 16 * t;
+        xeb[buf] = *reinterpret_cast<const float4*>(p);
+        xsb[buf] = *reinterpret_cast<const float4*>(p + MT);
+      };
+      scales(0, 0, 0);
+      {
+        const long bw = w.operand(0);
+#pragma unroll
+        for (int t = 0; t < WA; t++)
+          e[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(act(0, t), bw, base, 0, 0, 0);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        w.pin();  // (left alone, the compiler unpacks all eight sub-blocks first)
+        const float ds = dsj[j & 1], dm = dmj[j & 1], nds = -(ds * E_BASE);
+        long bw = 0;
+        if (j + 1 < 8) {
+          dsj[(j + 1) & 1] = from(j + 1, ds2);
+          dmj[(j + 1) & 1] = from(j + 1, dm2);
+          bw = w.operand(j + 1);
+        }
+#pragma unroll
+        for (int t = 0; t < WA; t++) {
+          const int st = j * WA + t, buf = st & 1;
+          long xa = 0;
+          if (j + 1 < 8) xa = act(j + 1, t);
+          if (st + 1 < 8 * WA) scales((st + 1) / WA, (st + 1) % WA, buf ^ 1);
+          __builtin_amdgcn_sched_barrier(0);
+          const float4 xe = xeb[buf], xs = xsb[buf];
+          const float xev[4] = {xe.x, xe.y, xe.z, xe.w}, xsv[4] = {xs.x, xs.y, xs.z, xs.w};
+          // the four terms side by side (left alone, the compiler forms one after
+          // the other, each operation waiting for the one before)
+          float se[4], dx[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            se[i] = FIN ? fmaf(ds, __int_as_float(e[t][i]), nds) : ds * (float)e[t][i];
+#pragma unroll
+          for (int i = 0; i < 4; i++) dx[i] = dm * xsv[i];
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < 4; i++) se[i] = se[i] - dx[i];
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < 4; i++) se[i] = xev[i] * se[i];
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < 4; i++) acc[t][i] += se[i];
+          // the next sub-block's sums run under the other tiles' terms
+          if (j + 1 < 8) e[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(xa, bw, base, 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    };
+    if (wild)
+      block(Bool<false>{});
+    else
+      block(Bool<true>{});
+  }
+  // this lane: weight row wr, activation rows 4 G .. + 3 of each tile
+  if (wr >= N) return;
+  const float bias = BIAS ? BIAS[wr] : 0.0f;
+#pragma unroll
+  for (int t = 0; t < WA; t++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t a = a0 + 16 * t + 4 * G + i;
+      if (a >= P.m) continue;
+      float* o = DST + (size_t)a * N + wr;
+      float v = acc[t][i];
+      if (BIAS) v = v + bias;
+      if (P.accum) v = *o + v;
+      *o = v;
+    }
 }
 
 // ------------------------------------------- 32-value blocks (Q8_0, Q5_0)
@@ -772,9 +1043,16 @@ Config make_config(gemm_kernel* k) {
   return Config{SH::TW, SH::MT, 64 * SH::NW, SH::lds(S)};
 }
 
+template <int T, int NW, int WA, int OCC>
+Config make_config_w(gemm_kernel* k) {
+  using SH = WShape<NW, WA>;
+  *k = k_gemm_w<T, NW, WA, OCC>;
+  return Config{SH::TW, SH::MT, 64 * NW, SH::lds};
+}
+
 // The tile shapes: weight rows x activation rows, waves, super-blocks per
-// stage, ring stages. Each is the fastest of a sweep for some (n, m) of
-// BASELINE config 4 (11008 x 2048 and 2048 x 11008, m = 2 .. 512).
+// stage, ring stages. 0 to 5 (k_gemm) are each the fastest of a sweep for some
+// (n, m) of 11008 x 2048 and 2048 x 11008, m = 2 .. 512; 6 to 8 are k_gemm_w.
 template <int T>
 Config config(int id, gemm_kernel* k) {
   switch (id) {
@@ -784,22 +1062,39 @@ Config config(int id, gemm_kernel* k) {
     case 3: return make_config<T, 4, 2, 1, 1, 2, 2>(k);  // 64 x 32, 8 waves
     case 4: return make_config<T, 2, 2, 1, 1, 2, 2>(k);  // 32 x 32
     case 5: return make_config<T, 4, 2, 2, 1, 1, 3>(k);  // 64 x 64, 8 waves
-    default: return make_config<T, 8, 1, 4, 1, 1, 2>(k);  // 128 x 64, 8 waves
+    case 6: return make_config_w<T, 4, 1, 4>(k);         // 64 x 16
+    case 7: return make_config_w<T, 4, 2, 4>(k);         // 64 x 32
+    default: return make_config_w<T, 4, 4, 3>(k);        // 64 x 64
   }
 }
 
-// Few weight rows (n < 4096: 2048 x 11008 and the q/o/k/v shapes) take the
-// largest tile (64 x 64, 64 x 32, then 32 x 32) that gives at least 5/8 of
-// the CUs a workgroup; below that, 16 x 16 tiles that split k over the
-// waves (four super-blocks a stage up to a workgroup per CU, two past it).
-// Swept at n = 2048 (k = 2048 and 11008) and n = 256 for m = 64 to 512: the
-// rule picks the fastest tile or one within 3% of it; at a prefill
-// chunk (m = 256) 2048 x 11008 takes 62 us in 64 x 32 tiles against 88 in
-// 64 x 64, 2048 x 2048 16.3 against 20.6, 256 x 2048 9.5 in 16 x 16 against
-// 20.8.
+// Weights in registers (k_gemm_w) where its tiles give the chip enough
+// workgroups, the larger tile first; measured against the best k_gemm tile, us:
+//   64 x 64: 11008 x 2048 m = 512 79, 83, m = 256 48, 57; 14336 x 4096 m = 512 161,
+//     181, m = 128 57, 64; 4096 x 4096 m = 512 62, 69
+//   64 x 32: 11008 x 2048 m = 128 34, 39; 4096 x 4096 m = 256 42, 63; 2048 x 11008
+//     m = 512 93, 100 (its 512 workgroups; at m = 256 79, 69: k_gemm)
+//   64 x 16: 4096 x 4096 m = 64 28, 40, m = 128 32, 62; 4096 x 14336 (Q5_K) m = 32
+//     78, 85; 2048 x 11008 m = 128 58, 55, 1847 x 2048 m = 389 38, 28: k_gemm
+// Otherwise, with m <= 16 rows of many weights, 64 x 16 of k_gemm (11008 x 2048 18.4
+// against 18.9), and for few weight rows (n < 4096: 2048 x 11008 and the q/o/k/v
+// shapes) the largest k_gemm tile (64 x 64, 64 x 32, then 32 x 32) that gives at
+// least 5/8 of the CUs a workgroup; below that, 16 x 16 tiles that split k over the
+// waves (four super-blocks a stage up to a workgroup per CU, two past it). Swept at
+// n = 2048 (k = 2048 and 11008) and n = 256 for m = 64 to 512: the rule picks the
+// fastest tile or one within 3% of it; at m = 256 2048 x 11008 takes 62 us in 64 x 32
+// tiles against 88 in 64 x 64, 2048 x 2048 16.3 against 20.6, 256 x 2048 9.5 in 16 x
+// 16 against 20.8.
 int choose(uint32_t n, uint32_t m) {
-  if (n >= 4096) return m <= 16 ? 2 : m <= 32 ? 3 : m <= 64 ? 5 : 6;
   auto tiles = [&](uint32_t tw, uint32_t mt) { return (n + tw - 1) / tw * ((m + mt - 1) / mt); };
+  const bool few = n < 4096;
+  if (m > 16) {
+    if (tiles(64, 64) >= (few ? 768u : 440u)) return 8;
+    if (tiles(64, 32) >= (few ? 512u : 300u)) return 7;
+    if (!few && tiles(64, 16) >= 128) return 6;
+  } else if (!few) {
+    return 2;
+  }
   constexpr uint32_t ENOUGH = 256 * 5 / 8;  // workgroups, on 256 CUs
   if (tiles(64, 64) >= ENOUGH) return 5;
   if (tiles(64, 32) >= ENOUGH) return 3;
