@@ -106,16 +106,16 @@ struct GemmParams {
   const float* xexs;    // per sub-block J: xe of the m_pad rows, then their xs
   float* dst;           // m x n
   uint32_t n, k, m, m_pad, nb, row_bytes, row_tiles, act_tiles;
-  const float* lhs;     // m x k f32: the quantizer's input (not read by k_gemm)
-  uint8_t* scratch;     // where xq and xexs are carved (not read by k_gemm)
-  // k_gemm only: with nseg > 1 the n rows are nseg matrices of one type and
+  const float* lhs;     // m x k f32: the quantizer's input (not read by the kernels)
+  uint8_t* scratch;     // where xq and xexs are carved (not read by the kernels)
+  // with nseg > 1 the n rows are nseg matrices of one type and
   // width, rows [sr[i], sr[i + 1]) matrix i with weights sw[i] and its own
   // output sd[i] (m x (sr[i + 1] - sr[i])); every sr[i] is a multiple of
   // the tile's rows, so a tile lies in one matrix
   uint32_t nseg, sr[CX_GEMM_SEGS + 1];
   const uint8_t* sw[CX_GEMM_SEGS];
   float* sd[CX_GEMM_SEGS];
-  // k_gemm only, per matrix (index 0 without segments): a bias added to
+  // per matrix (index 0 without segments): a bias added to
   // every output row (dst = acc + bias[r]), and with accum the output added
   // to what dst holds (dst = dst + (acc [+ bias])), f32 adds as written
   const float* sbias[CX_GEMM_SEGS];
@@ -448,6 +448,26 @@ template <int NW, int WA> struct WShape {
   static constexpr size_t lds = 2 * STAGE;
 };
 
+// the sums of one lane: weight row wr, activation rows 4 G .. + 3 of each tile from a0
+template <int WA>
+__device__ inline void store_rows(const GemmParams& P, const float (&acc)[WA][4], float* dst,
+                                  const float* bias, uint32_t n, uint32_t wr, uint32_t a0, int G) {
+  if (wr >= n) return;
+  const float bv = bias ? bias[wr] : 0.0f;
+#pragma unroll
+  for (int t = 0; t < WA; t++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t a = a0 + 16 * t + 4 * G + i;
+      if (a >= P.m) continue;
+      float* o = dst + (size_t)a * n + wr;
+      float v = acc[t][i];
+      if (bias) v = v + bv;
+      if (P.accum) v = *o + v;
+      *o = v;
+    }
+}
+
 template <int T, int NW, int WA, int OCC>
 __global__ __launch_bounds__(64 * NW, OCC) void k_gemm_w(GemmParams P) {
   static_assert(NW % 4 == 0, "a wave's loads are rows of one remainder mod 16");
@@ -622,322 +642,428 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_gemm_w(GemmParams P) {
     else
       block(Bool<true>{});
   }
-  // this lane: weight row wr, activation rows 4 G .. + 3 of each tile
-  if (wr >= N) return;
-  const float bias = BIAS ? BIAS[wr] : 0.0f;
-#pragma unroll
-  for (int t = 0; t < WA; t++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const uint32_t a = a0 + 16 * t + 4 * G + i;
-      if (a >= P.m) continue;
-      float* o = DST + (size_t)a * N + wr;
-      float v = acc[t][i];
-      if (BIAS) v = v + bias;
-      if (P.accum) v = *o + v;
-      *o = v;
-    }
+  store_rows<WA>(P, acc, DST, BIAS, N, wr, a0, G);
 }
 
-// ------------------------------------------- 32-value blocks (Q8_0, Q5_0)
-// The reference's buffer path (ops::matmul_i8_directo, src/ops.rs:310-414;
-// its m >= 24 blocked path adds in another order, src/ops.rs:726): one
-// v_mfma_i32_16x16x32_i8 per block gives a 16 (activation rows) x 16 (weight
-// rows) tile of exact block dots E; each lane applies the GEMV's term
-// (d * xe) * E to its four outputs and adds them block after block from 0,
-// so every output equals k_gemv32's bit for bit. A workgroup of 4 waves
-// covers 64 weight rows x 16 activation rows; the operands are read
-// straight from global memory (rows of 34- and 22-byte blocks sit at any
-// even offset: 16-bit loads), GB32_DEPTH blocks ahead of the MFMA.
-template <int T> struct GB;
-template <> struct GB<CX_Q8_0> {
-  static constexpr int BPB = 34;
-  struct Raw {
-    uint16_t d, q[4];
+// ---------------------------- the other formats (Q2_K, Q3_K, Q6_K, Q8_0, Q5_0)
+// The same layout and pipeline as k_gemm_w for the formats whose blocks sit at any
+// even offset of a row (84, 110 and 210 bytes of 256 values; 34 and 22 of 32):
+// XQ<T> holds one lane's share of a stage of 256 values of its weight row.
+//
+// A 32-value group is one v_mfma_i32_16x16x32_i8 for the 32-value formats (the
+// reference's buffer path, ops::matmul_i8_directo, src/ops.rs:310-414; its m >= 24
+// blocked path adds in another order, src/ops.rs:726). The others have two 16-value
+// sub-blocks in it: lanes of groups 0 and 1 hold the first, 2 and 3 the second, and
+// two MFMAs, each with the other half's weight bytes zero, give the two sums.
+//
+// The offsets that Q6_K (32), Q3_K (4) and Q5_0 (16) take off a value are taken off
+// its byte: the MFMA then sums E' = E - 32 xs itself, the exact integer that the
+// per-row kernel's (float)E - 32.0f * xs is, and the term is (xe * scale) * E' as
+// there. The MFMA starts from the bits of E_BASE, so that E' as f32 is one
+// subtraction at full rate, not a conversion at half (|E'| < 2^22: exact).
+typedef uint32_t u32_at2 __attribute__((aligned(2)));  // a word at any even address
+__device__ inline uint32_t at2(const uint8_t* p) { return *reinterpret_cast<const u32_at2*>(p); }
+__device__ inline uint2 at2x2(const uint8_t* p) {
+  struct __attribute__((packed, aligned(2))) Pair {
+    uint32_t x, y;
   };
-  // d and the quants at positions 8g .. 8g+7 of the block
-  __device__ static void load(const uint8_t* blk, int g, Raw& r) {
-    const uint16_t* h = reinterpret_cast<const uint16_t*>(blk);
-    r.d = h[0];
-#pragma unroll
-    for (int i = 0; i < 4; i++) r.q[i] = h[1 + 4 * g + i];
-  }
-  __device__ static long operand(const Raw& r, int) {
-    const uint32_t lo = (uint32_t)r.q[0] | ((uint32_t)r.q[1] << 16);
-    const uint32_t hi = (uint32_t)r.q[2] | ((uint32_t)r.q[3] << 16);
-    return (long)(((uint64_t)hi << 32) | lo);
-  }
-};
-template <> struct GB<CX_Q5_0> {
-  static constexpr int BPB = 22;
-  struct Raw {
-    uint16_t d, qh[2], qs[4];
-  };
-  // d, the fifth bits and the nibble bytes of positions 8g .. 8g+7: value
-  // i < 16 is the low nibble of qs[i], value 16 + i the high one
-  __device__ static void load(const uint8_t* blk, int g, Raw& r) {
-    const uint16_t* h = reinterpret_cast<const uint16_t*>(blk);
-    r.d = h[0];
-    r.qh[0] = h[1];
-    r.qh[1] = h[2];
-#pragma unroll
-    for (int i = 0; i < 4; i++) r.qs[i] = h[3 + 4 * (g & 1) + i];
-  }
-  __device__ static uint32_t spread4(uint32_t t) {  // bit i -> bit 4 of byte i
-    return ((t & 1u) << 4) | ((t & 2u) << 11) | ((t & 4u) << 18) | ((t & 8u) << 25);
-  }
-  __device__ static long operand(const Raw& r, int g) {
-    const uint32_t qh = (uint32_t)r.qh[0] | ((uint32_t)r.qh[1] << 16);
-    const uint32_t sh = g < 2 ? 0u : 4u;
-    const uint32_t w0 = ((uint32_t)r.qs[0] | ((uint32_t)r.qs[1] << 16)) >> sh;
-    const uint32_t w1 = ((uint32_t)r.qs[2] | ((uint32_t)r.qs[3] << 16)) >> sh;
-    const uint32_t t = (qh >> (8 * g)) & 0xFFu;
-    // (u - 16) in every byte, u in 0..31: biased by 128 so no byte borrows
-    const uint32_t lo = (((w0 & 0x0F0F0F0Fu) | spread4(t & 15u)) | 0x80808080u) - 0x10101010u;
-    const uint32_t hi = (((w1 & 0x0F0F0F0Fu) | spread4(t >> 4)) | 0x80808080u) - 0x10101010u;
-    return (long)(((uint64_t)(hi ^ 0x80808080u) << 32) | (lo ^ 0x80808080u));
-  }
-};
-
-constexpr int GB32_DEPTH = 4;
-
-template <int T>
-__global__ __launch_bounds__(256) void k_gemm32(GemmParams P) {
-  using Q = GB<T>;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 4, c16 = lane & 15;
-  // the activation tiles of one row tile share blockIdx % 8 (one XCD's L2)
-  const uint32_t b = blockIdx.x, A = P.act_tiles;
-  const uint32_t rt = b / (8 * A) * 8 + b % 8, at = b / 8 % A;
-  if (rt >= P.row_tiles) return;
-  const uint32_t r = rt * 64 + 16 * wave + c16;  // this lane's weight row (B column)
-  const uint32_t a0 = at * 16;
-  const uint8_t* wrow = P.w + (size_t)min(r, P.n - 1) * P.row_bytes;  // past the end: a valid row
-  const int8_t* xrow = P.xq + (size_t)(a0 + c16) * P.k + 8 * g;     // A operand: row a0 + c16
-  const float* xe = P.xexs + a0 + 4 * g;  // block J: xe of the tile's rows at J * 2 * m_pad
-  const uint32_t nb = P.k / 32;
-  typename Q::Raw wr[GB32_DEPTH];
-  long ax[GB32_DEPTH];
-  float4 xv[GB32_DEPTH];
-  auto fetch = [&](uint32_t j, int slot) {
-    Q::load(wrow + (size_t)j * Q::BPB, g, wr[slot]);
-    ax[slot] = *reinterpret_cast<const long*>(xrow + 32 * j);
-    xv[slot] = *reinterpret_cast<const float4*>(xe + (size_t)j * 2 * P.m_pad);
-  };
-#pragma unroll
-  for (int d = 0; d < GB32_DEPTH; d++)
-    if ((uint32_t)d < nb) fetch(d, d);
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (uint32_t j0 = 0; j0 < nb; j0 += GB32_DEPTH) {
-#pragma unroll
-    for (int d = 0; d < GB32_DEPTH; d++) {
-      const uint32_t j = j0 + d;
-      if (j < nb) {
-        v4i e = {0, 0, 0, 0};
-        e = __builtin_amdgcn_mfma_i32_16x16x32_i8(ax[d], Q::operand(wr[d], g), e, 0, 0, 0);
-        const float dw = cx_h2f(wr[d].d);
-        const float xs4[4] = {xv[d].x, xv[d].y, xv[d].z, xv[d].w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) acc[i] += dw * xs4[i] * (float)e[i];
-        if (j + GB32_DEPTH < nb) fetch(j + GB32_DEPTH, d);
-      }
-    }
-  }
-  if (r < P.n) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const uint32_t a = a0 + 4 * g + i;
-      if (a < P.m) P.dst[(size_t)a * P.n + r] = acc[i];
-    }
-  }
+  const Pair v = *reinterpret_cast<const Pair*>(p);
+  return make_uint2(v.x, v.y);
+}
+__device__ inline void pin(uint2& v) { asm volatile("" : "+v"(v.x), "+v"(v.y)); }
+__device__ inline uint2 both(uint2 v, uint32_t sh, uint32_t mask) {
+  return make_uint2((v.x >> sh) & mask, (v.y >> sh) & mask);
+}
+// every byte less `off`, as i8 (bytes <= 127 - (128 - off) before)
+__device__ inline uint2 less(uint2 v, uint32_t off) {
+  const uint32_t a = 0x01010101u * (128 - off);
+  return make_uint2((v.x + a) ^ 0x80808080u, (v.y + a) ^ 0x80808080u);
 }
 
-// ----------------------------- 16-value sub-blocks (Q2_K, Q3_K, Q6_K)
-// A 32-value group of a super-block holds two sub-blocks: lanes 16..31 of
-// the group's MFMA K range (lane groups g = 0, 1) are sub-block 2G and
-// 32..63 (g = 2, 3) sub-block 2G + 1. Two MFMAs per group, each with the
-// other sub-block's weight bytes zeroed, give the two exact sums; each lane
-// then applies the GEMV's term (k_gemv's KQ<T>) and adds in sub-block order,
-// so every output equals the per-row GEMV bit for bit. Operands come
-// straight from global memory (16-bit loads: 84-, 110- and 210-byte blocks
-// leave rows at any even offset).
-template <int T> struct GK;
-__device__ inline long pack8(uint32_t lo, uint32_t hi) {
-  return (long)(((uint64_t)hi << 32) | lo);
-}
-__device__ inline uint32_t w16(const uint16_t* h) { return (uint32_t)h[0] | ((uint32_t)h[1] << 16); }
+// Members: load(), this lane's words of the stage at p, of which `left` blocks are
+// in the row (a block past them reads the last); pin(); scales(), the factors of
+// this lane's sub-blocks PL G .. + PL (MIN: and their minima); operand(), its bytes
+// 8 G .. + 8 of the stage's 32-value group gg.
+template <int T> struct XQ;
 
 // Q2_K, 84 B: scales(16: low nibble scale, high nibble min) qs(64) d dmin;
-// value (qs[32(G/4) + i] >> 2(G%4)) & 3 (src/kernels/q2k.rs:41-69)
-template <> struct GK<CX_Q2_K> {
-  static constexpr int BPB = 84;
-  struct Raw {
-    uint16_t q[4], sc, d, dm;
-  };
-  __device__ static void load(const uint8_t* blk, int G, int g, Raw& r) {
-    const uint16_t* h = reinterpret_cast<const uint16_t*>(blk);
-    const int q0 = (16 + 32 * (G / 4) + 8 * g) / 2;
+// value (qs[32(gg/4) + i] >> 2(gg%4)) & 3 (src/kernels/q2k.rs:41-69)
+template <> struct XQ<CX_Q2_K> {
+  static constexpr int BPB = 84, SUB = 16, NB = 1, PL = 4;
+  static constexpr bool MIN = true;
+  uint2 q[2];
+  uint32_t sc, d;
+  __device__ void load(const uint8_t* p, int G, uint32_t) {
+    q[0] = at2x2(p + 16 + 8 * G);
+    q[1] = at2x2(p + 48 + 8 * G);
+    sc = at2(p + 4 * G);
+    d = at2(p + 80);
+  }
+  __device__ void pin() { ::pin(q[0]), ::pin(q[1]); }
+  __device__ void arrived() {
+    asm volatile("" : "+v"(sc), "+v"(d));
+    pin();
+  }
+  __device__ void scales(int, float (&s)[PL], float (&m)[PL]) const {
+    const float df = cx_h2f(d & 0xFFFFu), dm = cx_h2f(d >> 16);
 #pragma unroll
-    for (int i = 0; i < 4; i++) r.q[i] = h[q0 + i];
-    r.sc = h[G];  // the scale bytes of sub-blocks 2G, 2G+1
-    r.d = h[40];
-    r.dm = h[41];
+    for (int i = 0; i < PL; i++) {
+      s[i] = df * (float)((sc >> (8 * i)) & 15u);
+      m[i] = dm * (float)((sc >> (8 * i + 4)) & 15u);
+    }
   }
-  __device__ static long operand(const Raw& r, int G, int) {
-    const uint32_t sh = 2 * (G % 4);
-    return pack8((w16(r.q) >> sh) & 0x03030303u, (w16(r.q + 2) >> sh) & 0x03030303u);
-  }
-  __device__ static float term(const Raw& r, int G, int hf, int e, float xe, float xs) {
-    (void)G;
-    const uint32_t sc = hf ? (r.sc >> 8) : (r.sc & 0xFFu);
-    const float d = cx_h2f(r.d), dm = cx_h2f(r.dm);
-    return xe * (d * (float)(sc & 0xF) * (float)e - dm * (float)(sc >> 4) * xs);
-  }
+  __device__ uint2 operand(int gg, int) const { return both(q[gg / 4], 2 * (gg % 4), 0x03030303u); }
 };
 
 // Q3_K, 110 B: hmask(32) qs(64) scales(12) d; value (q + 4) =
-// ((qs[32(G/4) + i] >> 2(G%4)) & 3) | ((hmask[i] >> G) & 1) << 2
-// (src/kernels/scalar.rs:236-275), scales as quant::escalas_q3k
-template <> struct GK<CX_Q3_K> {
-  static constexpr int BPB = 110;
-  struct Raw {
-    uint16_t q[4], hm[4], sw[6], d;
-  };
-  __device__ static void load(const uint8_t* blk, int G, int g, Raw& r) {
-    const uint16_t* h = reinterpret_cast<const uint16_t*>(blk);
-    const int q0 = (32 + 32 * (G / 4) + 8 * g) / 2;
+// ((qs[32(gg/4) + i] >> 2(gg%4)) & 3) | ((hmask[i] >> gg) & 1) << 2
+// (src/kernels/scalar.rs:236-275), scales as quant::escalas_q3k (src/quant.rs:87-106)
+template <> struct XQ<CX_Q3_K> {
+  static constexpr int BPB = 110, SUB = 16, NB = 1, PL = 4;
+  static constexpr bool MIN = false;
+  uint2 q[2], h;
+  uint32_t s0, s1, s2, d;
+  __device__ void load(const uint8_t* p, int G, uint32_t) {
+    h = at2x2(p + 8 * G);
+    q[0] = at2x2(p + 32 + 8 * G);
+    q[1] = at2x2(p + 64 + 8 * G);
+    s0 = at2(p + 96);
+    s1 = at2(p + 100);
+    s2 = at2(p + 104);
+    d = *reinterpret_cast<const uint16_t*>(p + 108);
+  }
+  __device__ void pin() { ::pin(q[0]), ::pin(q[1]), ::pin(h); }
+  __device__ void arrived() {
+    asm volatile("" : "+v"(s0), "+v"(s1), "+v"(s2), "+v"(d));
+    pin();
+  }
+  __device__ void scales(int G, float (&s)[PL], float (&)[PL]) const {
+    const uint32_t low = ((G & 1 ? s1 : s0) >> (G & 2 ? 4 : 0)) & 0x0F0F0F0Fu;
+    const uint32_t w = low | (((s2 >> (2 * G)) & 0x03030303u) << 4);
+    const float df = cx_h2f(d);
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      r.q[i] = h[q0 + i];
-      r.hm[i] = h[4 * g + i];
-    }
-#pragma unroll
-    for (int i = 0; i < 6; i++) r.sw[i] = h[48 + i];
-    r.d = h[54];
+    for (int i = 0; i < PL; i++) s[i] = df * ((float)((w >> (8 * i)) & 63u) - 32.0f);
   }
-  __device__ static long operand(const Raw& r, int G, int) {
-    const uint32_t sh = 2 * (G % 4);
-    const uint32_t lo = ((w16(r.q) >> sh) & 0x03030303u) | (((w16(r.hm) >> G) & 0x01010101u) << 2);
-    const uint32_t hi =
-        ((w16(r.q + 2) >> sh) & 0x03030303u) | (((w16(r.hm + 2) >> G) & 0x01010101u) << 2);
-    return pack8(lo, hi);
-  }
-  // the 6-bit signed scale of sub-block s (src/quant.rs:87-106)
-  __device__ static float esc(const Raw& r, int s) {
-    const uint32_t m1 = 0x03030303u, m2 = 0x0F0F0F0Fu;
-    const uint32_t a0 = w16(r.sw), a1 = w16(r.sw + 2), t = w16(r.sw + 4);
-    uint32_t w;
-    switch (s / 4) {
-      case 0: w = (a0 & m2) | ((t & m1) << 4); break;
-      case 1: w = (a1 & m2) | (((t >> 2) & m1) << 4); break;
-      case 2: w = ((a0 >> 4) & m2) | (((t >> 4) & m1) << 4); break;
-      default: w = ((a1 >> 4) & m2) | (((t >> 6) & m1) << 4); break;
-    }
-    return (float)(int8_t)(uint8_t)(w >> (8 * (s % 4)));
-  }
-  __device__ static float term(const Raw& r, int G, int hf, int e, float xe, float xs) {
-    const float scale = cx_h2f(r.d) * (esc(r, 2 * G + hf) - 32.0f);
-    return xe * scale * ((float)e - 4.0f * xs);
+  __device__ uint2 operand(int gg, int) const {
+    const uint2 a = both(q[gg / 4], 2 * (gg % 4), 0x03030303u), b = both(h, gg, 0x01010101u);
+    return less(make_uint2(a.x | (b.x << 2), a.y | (b.y << 2)), 4);
   }
 };
 
-// Q6_K, 210 B: ql(128) qh(64) scales(16, i8) d. Group G: half = G/4,
-// gi = G%4; value = nibble | ((qh[32 half + i] >> 2gi) & 3) << 4, the nibble
-// low (gi < 2) or high of ql[64 half + 32 (gi%2) + i] (src/kernels/scalar.rs:294-324)
-template <> struct GK<CX_Q6_K> {
-  static constexpr int BPB = 210;
-  struct Raw {
-    uint16_t ql[4], qh[4], sc, d;
-  };
-  __device__ static void load(const uint8_t* blk, int G, int g, Raw& r) {
-    const uint16_t* h = reinterpret_cast<const uint16_t*>(blk);
-    const int half = G / 4, gi = G % 4;
-    const int l0 = (64 * half + 32 * (gi % 2) + 8 * g) / 2, h0 = (128 + 32 * half + 8 * g) / 2;
+// Q6_K, 210 B: ql(128) qh(64) scales(16, i8) d. Group gg: half = gg/4, gi = gg%4;
+// value = nibble | ((qh[32 half + i] >> 2gi) & 3) << 4, the nibble low (gi < 2) or
+// high of ql[64 half + 32 (gi%2) + i] (src/kernels/scalar.rs:294-324)
+template <> struct XQ<CX_Q6_K> {
+  static constexpr int BPB = 210, SUB = 16, NB = 1, PL = 4;
+  static constexpr bool MIN = false;
+  uint2 q[4], h[2];
+  uint32_t sc, d;
+  __device__ void load(const uint8_t* p, int G, uint32_t) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      r.ql[i] = h[l0 + i];
-      r.qh[i] = h[h0 + i];
-    }
-    r.sc = h[96 + G];
-    r.d = h[104];
+    for (int i = 0; i < 4; i++) q[i] = at2x2(p + 32 * i + 8 * G);
+    h[0] = at2x2(p + 128 + 8 * G);
+    h[1] = at2x2(p + 160 + 8 * G);
+    sc = at2(p + 192 + 4 * G);
+    d = *reinterpret_cast<const uint16_t*>(p + 208);
   }
-  __device__ static long operand(const Raw& r, int G, int) {
-    const int gi = G % 4;
-    const uint32_t ns = gi < 2 ? 0u : 4u, hs = 2 * gi;
-    const uint32_t lo = ((w16(r.ql) >> ns) & 0x0F0F0F0Fu) | (((w16(r.qh) >> hs) & 0x03030303u) << 4);
-    const uint32_t hi =
-        ((w16(r.ql + 2) >> ns) & 0x0F0F0F0Fu) | (((w16(r.qh + 2) >> hs) & 0x03030303u) << 4);
-    return pack8(lo, hi);
+  __device__ void pin() {
+    ::pin(q[0]), ::pin(q[1]), ::pin(q[2]), ::pin(q[3]), ::pin(h[0]), ::pin(h[1]);
   }
-  __device__ static float term(const Raw& r, int G, int hf, int e, float xe, float xs) {
-    (void)G;
-    const float scale = cx_h2f(r.d) * (float)(int8_t)(uint8_t)(hf ? (r.sc >> 8) : (r.sc & 0xFFu));
-    return xe * scale * ((float)e - 32.0f * xs);
+  __device__ void arrived() {
+    asm volatile("" : "+v"(sc), "+v"(d));
+    pin();
+  }
+  __device__ void scales(int, float (&s)[PL], float (&)[PL]) const {
+    const float df = cx_h2f(d);
+#pragma unroll
+    for (int i = 0; i < PL; i++) s[i] = df * (float)(int8_t)(uint8_t)(sc >> (8 * i));
+  }
+  __device__ uint2 operand(int gg, int) const {
+    const int half = gg / 4, gi = gg % 4;
+    const uint2 a = both(q[2 * half + gi % 2], gi < 2 ? 0 : 4, 0x0F0F0F0Fu);
+    const uint2 b = both(h[half], 2 * gi, 0x03030303u);
+    return less(make_uint2(a.x | (b.x << 4), a.y | (b.y << 4)), 32);
   }
 };
 
-constexpr int GK16_DEPTH = 3;
+// Q8_0, 34 B: d, 32 signed bytes
+template <> struct XQ<CX_Q8_0> {
+  static constexpr int BPB = 34, SUB = 32, NB = 8, PL = 2;
+  static constexpr bool MIN = false;
+  uint2 q[8];
+  uint32_t d[2];
+  __device__ void load(const uint8_t* p, int G, uint32_t left) {
+#pragma unroll
+    for (uint32_t i = 0; i < 8; i++)
+      q[i] = at2x2(p + (i < left ? i : left - 1) * BPB + 2 + 8 * G);
+#pragma unroll
+    for (uint32_t i = 0; i < 2; i++)
+      d[i] = *reinterpret_cast<const uint16_t*>(p + min(2 * G + i, left - 1) * BPB);
+  }
+  __device__ void pin() {
+#pragma unroll
+    for (int i = 0; i < 8; i++) ::pin(q[i]);
+  }
+  __device__ void arrived() {
+    asm volatile("" : "+v"(d[0]), "+v"(d[1]));
+    pin();
+  }
+  __device__ void scales(int, float (&s)[PL], float (&)[PL]) const {
+    s[0] = cx_h2f(d[0]);
+    s[1] = cx_h2f(d[1]);
+  }
+  __device__ uint2 operand(int gg, int) const { return q[gg]; }
+};
 
-template <int T>
-__global__ __launch_bounds__(256) void k_gemm16(GemmParams P) {
-  using Q = GK<T>;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 4, c16 = lane & 15;
+// Q5_0, 22 B: d, the fifth bits of the 32 values, their nibbles: value i < 16 is
+// the low nibble of byte i, value 16 + i the high one
+template <> struct XQ<CX_Q5_0> {
+  static constexpr int BPB = 22, SUB = 32, NB = 8, PL = 2;
+  static constexpr bool MIN = false;
+  uint2 q[8];
+  uint32_t h[8], d[2];
+  __device__ void load(const uint8_t* p, int G, uint32_t left) {
+#pragma unroll
+    for (uint32_t i = 0; i < 8; i++) {
+      const uint8_t* b = p + (i < left ? i : left - 1) * BPB;
+      q[i] = at2x2(b + 6 + 8 * (G & 1));
+      h[i] = b[2 + G];
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 2; i++)
+      d[i] = *reinterpret_cast<const uint16_t*>(p + min(2 * G + i, left - 1) * BPB);
+  }
+  __device__ void pin() {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      ::pin(q[i]);
+      asm volatile("" : "+v"(h[i]));
+    }
+  }
+  __device__ void arrived() {
+    asm volatile("" : "+v"(d[0]), "+v"(d[1]));
+    pin();
+  }
+  __device__ void scales(int, float (&s)[PL], float (&)[PL]) const {
+    s[0] = cx_h2f(d[0]);
+    s[1] = cx_h2f(d[1]);
+  }
+  // bit i of a nibble to bit 4 of byte i
+  __device__ static uint32_t spread4(uint32_t t) {
+    return ((t & 1u) << 4) | ((t & 2u) << 11) | ((t & 4u) << 18) | ((t & 8u) << 25);
+  }
+  __device__ uint2 operand(int gg, int G) const {
+    const uint2 a = both(q[gg], G < 2 ? 0 : 4, 0x0F0F0F0Fu);
+    return less(make_uint2(a.x | spread4(h[gg] & 15u), a.y | spread4(h[gg] >> 4)), 16);
+  }
+};
+
+template <int T, int WA> struct XShape {
+  static constexpr int TW = 64, MT = 16 * WA;
+  static constexpr int NS = 256 / XQ<T>::SUB;      // sub-blocks a stage
+  static constexpr int PARTS = XQ<T>::MIN ? 2 : 1;  // xe, with minima xs too
+  static constexpr int ROW = PARTS * MT / 4;        // 16-byte chunks of a sub-block's xe (, xs)
+  // 1 KiB loads a stage: the activation rows; their xe (, xs)
+  static constexpr int LX = 4 * WA, LE = (NS * ROW + 63) / 64;
+  static constexpr int STAGE = (LX + LE) * 1024;
+  static constexpr size_t lds = 2 * STAGE;
+};
+
+template <int T, int WA, int OCC>
+__global__ __launch_bounds__(256, OCC) void k_gemm_x(GemmParams P) {
+  using Q = XQ<T>;
+  using SH = XShape<T, WA>;
+  constexpr int TW = SH::TW, MT = SH::MT, LX = SH::LX, LE = SH::LE, NS = SH::NS, NH = 32 / Q::SUB;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane % 16, G = lane / 16;
+  // blockIdx -> (row tile, activation tile), as k_gemm
   const uint32_t b = blockIdx.x, A = P.act_tiles;
   const uint32_t rt = b / (8 * A) * 8 + b % 8, at = b / 8 % A;
-  if (rt >= P.row_tiles) return;
-  const uint32_t r = rt * 64 + 16 * wave + c16;
-  const uint32_t a0 = at * 16;
-  const uint8_t* wrow = P.w + (size_t)min(r, P.n - 1) * P.row_bytes;
-  const int8_t* xrow = P.xq + (size_t)(a0 + c16) * P.k + 8 * g;
-  const float* xe = P.xexs + a0 + 4 * g;  // sub-block J: xe at J * 2 * m_pad, xs m_pad after
-  const uint32_t ng = P.k / 32;          // 32-value groups
-  typename Q::Raw wr[GK16_DEPTH];
-  long ax[GK16_DEPTH];
-  float4 xv[GK16_DEPTH][4];  // xe, xs of sub-block 2j, then of 2j + 1
-  auto fetch = [&](uint32_t j, int slot) {
-    Q::load(wrow + (size_t)(j / 8) * Q::BPB, (int)(j % 8), g, wr[slot]);
-    ax[slot] = *reinterpret_cast<const long*>(xrow + 32 * j);
+  if (rt >= P.row_tiles) return;  // whole workgroup, before any load or barrier
+  const uint32_t a0 = at * MT;
+  const uint8_t* W = P.w;
+  float* DST = P.dst;
+  const float* BIAS = P.sbias[0];
+  uint32_t N = P.n, r0 = rt * TW;
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const float* e = xe + (size_t)(2 * j + h) * 2 * P.m_pad;
-      xv[slot][2 * h] = *reinterpret_cast<const float4*>(e);
-      xv[slot][2 * h + 1] = *reinterpret_cast<const float4*>(e + P.m_pad);
+  for (uint32_t i = 0; i < CX_GEMM_SEGS; i++)
+    if (i < P.nseg && rt * TW >= P.sr[i]) {
+      W = P.sw[i];
+      DST = P.sd[i];
+      BIAS = P.sbias[i];
+      N = P.sr[i + 1] - P.sr[i];
+      r0 = rt * TW - P.sr[i];
+    }
+  r0 += 16 * wave;
+  const uint32_t wr = r0 + col;  // this lane's weight row (past the end: a valid row)
+  const uint8_t* wrow = W + (size_t)(wr < N ? wr : N - 1) * P.row_bytes;
+  // the loads of a stage as k_gemm_w's; in the row's last stage a chunk past k, and
+  // past the last sub-block, reads the stage's first one again (no term uses it)
+  const uint32_t xr = (lane / 16) * P.k, xc = 16 * ((lane % 16) ^ ((4 * wave + lane / 16) % 16));
+  const int8_t* xbase = P.xq + (size_t)a0 * P.k;
+  const float* ebase = P.xexs + a0;
+  const uint32_t nst = (P.nb + Q::NB - 1) / Q::NB;
+  auto issue = [&](uint32_t sb) {
+    uint8_t* l = lds + (sb & 1) * SH::STAGE;
+    const uint32_t left = P.k - 256 * sb;  // values
+    const uint32_t xoff = xr + (Q::NB == 1 || xc < left ? xc : 0u);
+#pragma unroll
+    for (int u = 0; u < LX / 4; u++) {
+      const int i = wave + 4 * u;
+      cx_dma16_async_s(xbase + (size_t)(4 * i) * P.k + 256 * sb, xoff, l + 1024 * i);
+    }
+#pragma unroll
+    for (int u = 0; u < (LE + 3) / 4; u++) {
+      const int i = wave + 4 * u;
+      if (i < LE) {
+        const uint32_t c = 64 * i + lane;  // chunk: sub-block c / ROW
+        uint32_t s = c / SH::ROW;
+        if (s >= (uint32_t)NS || (Q::NB > 1 && Q::SUB * s >= left)) s = 0;
+        const uint32_t eoff =
+            (2 * s + c % SH::ROW / (MT / 4)) * P.m_pad * 4 + 16 * (c % (MT / 4));
+        cx_dma16_async_s(ebase + (size_t)sb * (2 * NS) * P.m_pad, eoff, l + 1024 * (LX + i));
+      }
     }
   };
+  float acc[WA][4];
 #pragma unroll
-  for (int d = 0; d < GK16_DEPTH; d++)
-    if ((uint32_t)d < ng) fetch(d, d);
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (uint32_t j0 = 0; j0 < ng; j0 += GK16_DEPTH) {
+  for (int t = 0; t < WA; t++)
 #pragma unroll
-    for (int d = 0; d < GK16_DEPTH; d++) {
-      const uint32_t j = j0 + d;
-      if (j < ng) {
-        const int G = (int)(j % 8);
-        const long bw = Q::operand(wr[d], G, g);
-        v4i e0 = {0, 0, 0, 0}, e1 = {0, 0, 0, 0};
-        e0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(ax[d], g < 2 ? bw : 0l, e0, 0, 0, 0);
-        e1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(ax[d], g < 2 ? 0l : bw, e1, 0, 0, 0);
-        const float4 xe0 = xv[d][0], xs0 = xv[d][1], xe1 = xv[d][2], xs1 = xv[d][3];
-        const float a_e0[4] = {xe0.x, xe0.y, xe0.z, xe0.w}, a_s0[4] = {xs0.x, xs0.y, xs0.z, xs0.w};
-        const float a_e1[4] = {xe1.x, xe1.y, xe1.z, xe1.w}, a_s1[4] = {xs1.x, xs1.y, xs1.z, xs1.w};
+    for (int i = 0; i < 4; i++) acc[t][i] = 0.0f;
+  Q wn;
+  wn.load(wrow, G, P.nb);
+  issue(0);
+  const uint32_t half = G < 2 ? ~0u : 0u;  // (16-value sub-blocks)
+#pragma unroll 1
+  for (uint32_t sb = 0; sb < nst; sb++) {
+    cx_wait_vm<0>();  // this wave's part of stage sb, and its weights
+    cx_wait_lds();
+    cx_barrier();     // every wave's part; stage sb - 1 is read
+    Q w = wn;
+    w.arrived();  // before the next loads are issued, as in k_gemm_w
+    if (sb + 1 < nst) issue(sb + 1);
+    const uint32_t sn = sb + 1 < nst ? sb + 1 : sb;
+    wn.load(wrow + (size_t)sn * (Q::NB * Q::BPB), G, P.nb - sn * Q::NB);
+    const uint8_t* X = lds + (sb & 1) * SH::STAGE;
+    const float* E = reinterpret_cast<const float*>(X + 256 * MT) + 4 * G;
+    const uint32_t ng = Q::NB == 1 ? 8 : P.nb - sb * Q::NB;  // 32-value groups (more than 8: 8)
+    float sv[Q::PL], mv[Q::PL];
+    w.scales(G, sv, mv);
+    uint32_t ax = 256 * col + 16 * ((G / 2) ^ col) + 8 * (G & 1);
+    asm volatile("" : "+v"(ax));
+    auto act = [&](int gg, int t) {
+      return *reinterpret_cast<const long*>(X + (ax ^ (32 * gg)) + 4096 * t);
+    };
+    auto from = [&](int j, const float (&v)[Q::PL]) {  // this row's value for sub-block j
+      return __int_as_float(__builtin_amdgcn_ds_bpermute(4 * col + 64 * (j / Q::PL),
+                                                         __float_as_int(v[j % Q::PL])));
+    };
+    // the weight operands of group gg: one, or one per sub-block
+    auto operands = [&](int gg, long (&o)[NH]) {
+      const uint2 v = w.operand(gg, G);
+      if constexpr (NH == 1) {
+        o[0] = (long)(((uint64_t)v.y << 32) | v.x);
+      } else {
+        o[0] = (long)(((uint64_t)(v.y & half) << 32) | (v.x & half));
+        o[1] = (long)(((uint64_t)(v.y & ~half) << 32) | (v.x & ~half));
+      }
+    };
+    v4i base;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          acc[i] += Q::term(wr[d], G, 0, e0[i], a_e0[i], a_s0[i]);
-          acc[i] += Q::term(wr[d], G, 1, e1[i], a_e1[i], a_s1[i]);
+    for (int i = 0; i < 4; i++) base[i] = E_BASE_BITS;
+    v4i e[WA][NH];
+    float dsj[2][NH], dmj[2][NH];
+    auto factors = [&](int gg) {
+#pragma unroll
+      for (int h = 0; h < NH; h++) {
+        dsj[gg & 1][h] = from(NH * gg + h, sv);
+        if constexpr (Q::MIN) dmj[gg & 1][h] = from(NH * gg + h, mv);
+      }
+    };
+    // xe (, xs) of a tile's four activation rows, the next tile's read under this
+    // one's terms
+    float4 xeb[2], xsb[2];
+    auto scales = [&](int st) {  // st = (gg * WA + t) * NH + h
+      const int h = st % NH, t = st / NH % WA, gg = st / NH / WA;
+      const float* p = E + SH::PARTS * MT * (NH * gg + h) + 16 * t;
+      xeb[st & 1] = *reinterpret_cast<const float4*>(p);
+      if constexpr (Q::MIN) xsb[st & 1] = *reinterpret_cast<const float4*>(p + MT);
+    };
+    factors(0);
+    scales(0);
+    {
+      long bw[NH];
+      operands(0, bw);
+#pragma unroll
+      for (int t = 0; t < WA; t++)
+#pragma unroll
+        for (int h = 0; h < NH; h++)
+          e[t][h] = __builtin_amdgcn_mfma_i32_16x16x32_i8(act(0, t), bw[h], base, 0, 0, 0);
+    }
+#pragma unroll
+    for (int gg = 0; gg < 8; gg++) {
+      if (Q::NB > 1 && (uint32_t)gg >= ng) break;
+      w.pin();
+      long bw[NH];
+      if (gg + 1 < 8) {
+        factors(gg + 1);
+        operands(gg + 1, bw);
+      }
+#pragma unroll
+      for (int t = 0; t < WA; t++) {
+        long xa = 0;
+        if (gg + 1 < 8) xa = act(gg + 1, t);
+#pragma unroll
+        for (int h = 0; h < NH; h++) {
+          const int st = (gg * WA + t) * NH + h;
+          if (st + 1 < 8 * WA * NH) scales(st + 1);
+          __builtin_amdgcn_sched_barrier(0);
+          const float ds = dsj[gg & 1][h];
+          const float4 xe = xeb[st & 1];
+          const float xev[4] = {xe.x, xe.y, xe.z, xe.w};
+          float se[4], tx[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++) se[i] = __int_as_float(e[t][h][i]) - E_BASE;
+          if constexpr (Q::MIN) {  // xe * (d * sc * E - dmin * mn * xs)
+            const float dm = dmj[gg & 1][h];
+            const float4 xs = xsb[st & 1];
+            const float xsv[4] = {xs.x, xs.y, xs.z, xs.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++) tx[i] = dm * xsv[i];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) se[i] = ds * se[i];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) se[i] = se[i] - tx[i];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) se[i] = xev[i] * se[i];
+          } else {  // (xe * scale) * E'
+#pragma unroll
+            for (int i = 0; i < 4; i++) tx[i] = xev[i] * ds;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) se[i] = tx[i] * se[i];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < 4; i++) acc[t][i] += se[i];
+          if (gg + 1 < 8)
+            e[t][h] = __builtin_amdgcn_mfma_i32_16x16x32_i8(xa, bw[h], base, 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        if (j + GK16_DEPTH < ng) fetch(j + GK16_DEPTH, d);
+      }
+      if (Q::NB > 1) {  // (a branch follows: the adds stay on this side of it)
+#pragma unroll
+        for (int t = 0; t < WA; t++)
+          asm volatile("" : "+v"(acc[t][0]), "+v"(acc[t][1]), "+v"(acc[t][2]), "+v"(acc[t][3]));
       }
     }
   }
-  if (r < P.n) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const uint32_t a = a0 + 4 * g + i;
-      if (a < P.m) P.dst[(size_t)a * P.n + r] = acc[i];
-    }
-  }
+  store_rows<WA>(P, acc, DST, BIAS, N, wr, a0, G);
 }
 
 // ops::cuantizar_i8_en (src/ops.rs:178-198) of m rows into the layout above:
@@ -1122,12 +1248,55 @@ int quantize(const float* lhs, uint32_t m, uint32_t k, uint32_t m_pad, int sub, 
   return CX_OK;
 }
 
+// every tile height (16, 32 or 64 rows) divides 64
+inline uint32_t pad64(size_t m) { return (uint32_t)((m + 63) / 64 * 64); }
+
+// the formats of k_gemm_x
+bool direct_type(int type) { return cx_is_block32(type) || cx_sub(type) == 16; }
+
+template <int T, int WA, int OCC>
+Config make_config_x(gemm_kernel* k) {
+  using SH = XShape<T, WA>;
+  *k = k_gemm_x<T, WA, OCC>;
+  return Config{SH::TW, SH::MT, 256, SH::lds};
+}
+
+// The largest tile whose workgroups still keep the chip busy; us with 16, 32, 64
+// activation rows a workgroup (Q6_K, then Q8_0 whose term is shorter):
+//   Q6_K 4096 x 14336 m = 512 460, 303, 276, m = 256 249, 179, 209; 11008 x 2048
+//   m = 128 59, 45, 48, m = 17 28, 29, 38; 2048 x 11008 m = 256 137, 118, 165,
+//   m = 128 87, 112, 162
+//   Q8_0 4864 x 896 m = 512 56, 38, 32, m = 128 24, 22, 22; 2048 x 2048 m = 512 67,
+//   43, 33, m = 256 40, 29, 32, m = 128 27, 27, 31; 896 x 4864 m = 512 62, 50, 61
+template <int T>
+Config config_x(uint32_t n, uint32_t m, gemm_kernel* k) {
+  auto tiles = [&](uint32_t mt) { return (n + 63) / 64 * ((m + mt - 1) / mt); };
+  if (tiles(64) >= (XQ<T>::SUB == 32 ? 256u : 440u)) return make_config_x<T, 4, 3>(k);
+  if (tiles(32) >= 160u) return make_config_x<T, 2, 4>(k);
+  return make_config_x<T, 1, 4>(k);
+}
+Config config_x(int type, uint32_t n, uint32_t m, gemm_kernel* k) {
+  switch (type) {
+    case CX_Q8_0: return config_x<CX_Q8_0>(n, m, k);
+    case CX_Q5_0: return config_x<CX_Q5_0>(n, m, k);
+    case CX_Q2_K: return config_x<CX_Q2_K>(n, m, k);
+    case CX_Q3_K: return config_x<CX_Q3_K>(n, m, k);
+    default: return config_x<CX_Q6_K>(n, m, k);
+  }
+}
+
+// the tile of n weight rows of a type x m activation rows
+Config config_of(int type, uint32_t n, uint32_t m, gemm_kernel* k) {
+  if (type == CX_Q4_K) return config<CX_Q4_K>(choose(n, m), k);
+  if (type == CX_Q5_K) return config<CX_Q5_K>(choose(n, m), k);
+  return config_x(type, n, m, k);
+}
+
 // the contraction over rows quantized with a row count m_pad that is a
 // multiple of the chosen tile's height
-template <int T>
-int contract(GemmParams& P, hipStream_t s) {
+int contract(int type, GemmParams& P, hipStream_t s) {
   gemm_kernel k = nullptr;
-  const Config c = config<T>(choose(P.n, P.m), &k);
+  const Config c = config_of(type, P.n, P.m, &k);
   CX_REQUIRE(P.m_pad % c.mt == 0 && P.m_pad >= P.m, "gemm: %u padded rows for tiles of %d",
              P.m_pad, c.mt);
   P.xq = scratch_xq(P.scratch);
@@ -1140,42 +1309,6 @@ int contract(GemmParams& P, hipStream_t s) {
   CX_HIP(hipGetLastError());
   return CX_OK;
 }
-
-template <int T>
-int launch(GemmParams& P, hipStream_t s) {
-  gemm_kernel k = nullptr;
-  const Config c = config<T>(choose(P.n, P.m), &k);
-  // activation rows padded to the tile height (zero rows quantize to zero)
-  P.m_pad = (P.m + c.mt - 1) / c.mt * c.mt;
-  int rc = quantize(P.lhs, P.m, P.k, P.m_pad, 32, P.scratch, s);
-  return rc ? rc : contract<T>(P, s);
-}
-
-// every tile height (16, 32 or 64 rows) divides 64
-inline uint32_t pad64(size_t m) { return (uint32_t)((m + 63) / 64 * 64); }
-
-// the direct-operand contractions (32-value blocks and 16-value sub-blocks)
-// over rows quantized in scratch with the type's sub-block size (m_pad set)
-bool direct_type(int type) { return cx_is_block32(type) || cx_sub(type) == 16; }
-int contract_direct(int type, GemmParams& P, hipStream_t s) {
-  P.xq = scratch_xq(P.scratch);
-  P.xexs = scratch_xexs(P.scratch, P.m_pad, P.k);
-  P.row_tiles = (P.n + 63) / 64;
-  P.act_tiles = (P.m + 15) / 16;
-  const size_t grid = (size_t)(P.row_tiles + 7) / 8 * 8 * P.act_tiles;
-  CX_REQUIRE(grid < (1ull << 31), "gemm: %u x %u is too large", P.n, P.m);
-  const dim3 G((unsigned)grid), W(256);
-  switch (type) {
-    case CX_Q8_0: hipLaunchKernelGGL(k_gemm32<CX_Q8_0>, G, W, 0, s, P); break;
-    case CX_Q5_0: hipLaunchKernelGGL(k_gemm32<CX_Q5_0>, G, W, 0, s, P); break;
-    case CX_Q2_K: hipLaunchKernelGGL(k_gemm16<CX_Q2_K>, G, W, 0, s, P); break;
-    case CX_Q3_K: hipLaunchKernelGGL(k_gemm16<CX_Q3_K>, G, W, 0, s, P); break;
-    default: hipLaunchKernelGGL(k_gemm16<CX_Q6_K>, G, W, 0, s, P); break;
-  }
-  CX_HIP(hipGetLastError());
-  return CX_OK;
-}
-
 }  // namespace
 
 bool cx_gemm_supported(int type) { return cx_has_gemv(type); }
@@ -1206,12 +1339,12 @@ int cx_launch_gemm(int type, const uint8_t* w, size_t n, size_t k, const float* 
   P.m = (uint32_t)m;
   P.nb = (uint32_t)(k / vpb);
   P.row_bytes = P.nb * cx_bpb(type);
-  if (direct_type(type)) {
-    P.m_pad = pad64(m);
-    const int rc = quantize(lhs, P.m, P.k, P.m_pad, cx_sub(type), P.scratch, s);
-    return rc ? rc : contract_direct(type, P, s);
-  }
-  return type == CX_Q4_K ? launch<CX_Q4_K>(P, s) : launch<CX_Q5_K>(P, s);
+  // activation rows padded to the tile height (zero rows quantize to zero)
+  gemm_kernel kern = nullptr;
+  const uint32_t mt = (uint32_t)config_of(type, P.n, P.m, &kern).mt;
+  P.m_pad = (P.m + mt - 1) / mt * mt;
+  const int rc = quantize(lhs, P.m, P.k, P.m_pad, cx_sub(type), P.scratch, s);
+  return rc ? rc : contract(type, P, s);
 }
 
 int cx_gemm_quantize(const float* lhs, size_t m, size_t k, int sub, void* scratch, hipStream_t s) {
@@ -1289,20 +1422,18 @@ int cx_gemm_apply(int type, const uint8_t* w, size_t n, size_t k, size_t m, floa
   P.m_pad = pad64(m);
   P.nb = (uint32_t)(k / vpb);
   P.row_bytes = P.nb * cx_bpb(type);
-  if (direct_type(type)) return contract_direct(type, P, s);
-  return type == CX_Q4_K ? contract<CX_Q4_K>(P, s) : contract<CX_Q5_K>(P, s);
+  return contract(type, P, s);
 }
 
 bool cx_gemm_multi_fits(int type, const uint32_t* n, uint32_t count, size_t m) {
   if (!n || count < 1 || count > CX_GEMM_SEGS || !m || m >= (1u << 24) ||
-      !cx_gemm_supported(type) || direct_type(type))
+      !cx_gemm_supported(type))
     return false;
   uint32_t total = 0;
   for (uint32_t i = 0; i < count; i++) total += n[i];
   if (!total) return false;
   gemm_kernel kern = nullptr;
-  const Config c = type == CX_Q4_K ? config<CX_Q4_K>(choose(total, (uint32_t)m), &kern)
-                                   : config<CX_Q5_K>(choose(total, (uint32_t)m), &kern);
+  const Config c = config_of(type, total, (uint32_t)m, &kern);
   for (uint32_t i = 0; count > 1 && i < count; i++)
     if (n[i] % c.tw != 0) return false;  // a tile would straddle two matrices
   return true;
@@ -1320,8 +1451,8 @@ int cx_gemm_apply_multi(int type, const uint8_t* const* w, const uint32_t* n, ui
   P.scratch = const_cast<uint8_t*>(reinterpret_cast<const uint8_t*>(scratch));
   P.nseg = count;
   for (uint32_t i = 0; i < count; i++) {
-    CX_REQUIRE(w[i] && dst[i] && ((uintptr_t)w[i] & 15) == 0,
-               "gemm: matrix %u: null or misaligned (16-byte) pointer", i);
+    CX_REQUIRE(w[i] && dst[i] && ((uintptr_t)w[i] & (direct_type(type) ? 1 : 15)) == 0,
+               "gemm: matrix %u: null or misaligned (Q4_K/Q5_K 16-byte, others 2-byte) pointer", i);
     P.sw[i] = w[i];
     P.sd[i] = dst[i];
     P.sbias[i] = bias ? bias[i] : nullptr;
@@ -1336,5 +1467,5 @@ int cx_gemm_apply_multi(int type, const uint8_t* const* w, const uint32_t* n, ui
   P.m_pad = pad64(m);
   P.nb = (uint32_t)(k / vpb);
   P.row_bytes = P.nb * cx_bpb(type);
-  return type == CX_Q4_K ? contract<CX_Q4_K>(P, s) : contract<CX_Q5_K>(P, s);
+  return contract(type, P, s);
 }

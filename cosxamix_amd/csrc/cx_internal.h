@@ -179,7 +179,7 @@ int cx_gemm_apply(int type, const uint8_t* w, size_t n, size_t k, size_t m, floa
 // w[i]) into dst[i] (m x n[i]), with optional per-matrix biases (dst =
 // acc + bias[r]) and, with accum, added into dst (dst = dst + ...); every
 // value as cx_gemm_apply (and the separate adds) give it. Only where
-// cx_gemm_multi_fits: Q4_K/Q5_K, and with several matrices every n[i] a
+// cx_gemm_multi_fits: a type of cx_gemm_supported, and with several matrices every n[i] a
 // multiple of the tile's rows.
 #define CX_GEMM_SEGS 3
 bool cx_gemm_multi_fits(int type, const uint32_t* n, uint32_t count, size_t m);
