@@ -26,10 +26,10 @@
 //   k_samp_z     z_i and per-block maxima                      (grid)
 //   k_samp_e     e_i = exp(z_i - max), or the uniform 1/n       (grid)
 //   k_samp_sum   S sequentially, 1/S, and the draw of u         (1 workgroup)
-//   k_samp_p     p_i = e_i * (1/S)                              (grid)
-//   k_rs_count, k_rs_scan, k_rs_scatter, four times: the descending order
-//                of p (8-bit digits, least significant first); they return
-//                at once when top_p >= 1 (no order needed)
+//   k_rs_count, k_rs_scatter, four times: the descending order of p (8-bit
+//                digits, least significant first); the first count forms
+//                p_i = e_i * (1/S) as it reads e, and the rest returns at
+//                once when top_p >= 1 (no order needed)
 //   k_samp_pick  the token                                      (1 workgroup)
 // The sequential sums (S, the running sums) are ordered f32 sums that one
 // wave forms by binade scans (cx_scan.h), fed from LDS stages that the other
@@ -86,31 +86,23 @@ __global__ __launch_bounds__(ZB) void k_samp_z(const float* logits, uint32_t n,
 
 __global__ __launch_bounds__(ZB) void k_samp_e(float* pb, uint32_t n, const float* part,
                                                uint32_t nparts, cx_samp_state* sd) {
-  __shared__ float mx;
-  if (threadIdx.x == 0) {  // max over every z, NaN ignored (f32::max), from -inf
-    float m = -INFINITY;
-    for (uint32_t b = 0; b < nparts; b++) m = fmaxf(m, part[b]);
-    mx = m;
-    if (blockIdx.x == 0) sd->uniform = isfinite(m) ? 0u : 1u;
-  }
+  __shared__ float red[ZB / 64];
+  // max over every z, NaN ignored (f32::max), from -inf: the maxima a thread
+  // each (one thread's loop over 75 of them was a chain of loads)
+  float m = -INFINITY;
+  for (uint32_t b = threadIdx.x; b < nparts; b += ZB) m = fmaxf(m, part[b]);
+  m = cx_wave_max(m);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
-  const float m = mx;
+  m = red[0];
+  for (uint32_t w = 1; w < ZB / 64; w++) m = fmaxf(m, red[w]);
+  if (blockIdx.x == 0 && threadIdx.x == 0) sd->uniform = isfinite(m) ? 0u : 1u;
   const bool uni = !isfinite(m);
   const float u = 1.0f / (float)n;
   const uint32_t i0 = (blockIdx.x * ZB + threadIdx.x) * ZV;
   for (uint32_t j = 0; j < ZV; j++) {
     const uint32_t i = i0 + j;
     if (i < n) pb[i] = uni ? u : cx_expf(pb[i] - m);
-  }
-}
-
-__global__ __launch_bounds__(ZB) void k_samp_p(float* pb, uint32_t n, const cx_samp_state* sd) {
-  if (sd->uniform) return;  // the uniform probabilities are already in place
-  const float inv = sd->inv_s;
-  const uint32_t i0 = (blockIdx.x * ZB + threadIdx.x) * ZV;
-  for (uint32_t j = 0; j < ZV; j++) {
-    const uint32_t i = i0 + j;
-    if (i < n) pb[i] = pb[i] * inv;
   }
 }
 
@@ -350,20 +342,28 @@ __global__ __launch_bounds__(CW) void k_samp_sum(const float* pb, uint32_t n, cx
 // A stable LSD radix sort of (key, index) with key = ~total-order key of p:
 // ascending keys are descending probabilities (f32::total_cmp), and equal
 // ones keep ascending index. Four passes of 8-bit digits; a pass counts the
-// digits of each tile of RS_TILE elements, scans the counts (digit-major,
-// then tile), and scatters each tile in index order. Pass 0 reads p itself;
-// the last pass writes the order (ord) and the sorted probabilities (ordp).
+// digits of each tile of RS_TILE elements and scatters each tile in index
+// order, to offsets that are the counts' exclusive sums (digit-major, then
+// tile). Up to RS_SELF tiles (counts tile-major) each scatter workgroup sums
+// the counts it needs itself; above, where that would read tiles^2 counts,
+// k_rs_scan forms the offsets in place (counts digit-major) between the two.
+// Pass 0 forms p; the last pass writes the order (ord) and the sorted
+// probabilities (ordp).
+// (a scatter reads 1 KiB a tile for its offsets: 75 KiB at 151936 tokens)
+constexpr uint32_t RS_SELF = 128;
 __device__ inline uint32_t rs_key(float p) { return ~pkey(p); }
 __device__ inline float rs_p(uint32_t key) {  // the probability back from its key
   const uint32_t k = ~key;
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
 }
 
+// pb: in pass 0 the exps on entry (the uniform p where sd->uniform), p on return
 template <int D>
-__global__ __launch_bounds__(RS_T) void k_rs_count(const float* pb, const uint32_t* kin, uint32_t n,
+__global__ __launch_bounds__(RS_T) void k_rs_count(float* pb, const uint32_t* kin, uint32_t n,
                                                    const cx_samp_state* sd, uint32_t* cnt,
                                                    uint32_t G) {
-  if (sd->top_p >= 1.0f) return;
+  const bool sorts = !(sd->top_p >= 1.0f);
+  if (D != 0 && !sorts) return;
   __shared__ uint32_t h[256];
   const uint32_t tid = threadIdx.x, base = blockIdx.x * RS_TILE;
   h[tid] = 0;
@@ -371,45 +371,42 @@ __global__ __launch_bounds__(RS_T) void k_rs_count(const float* pb, const uint32
   // reads element n - 1 and is not counted); a load a round waited for
   // each in turn
   uint32_t key[RS_R];
+  if (D == 0) {
+    const float inv = sd->uniform ? 1.0f : sd->inv_s;  // (the uniform p is in place)
+    float p[RS_R];
 #pragma unroll
-  for (uint32_t r = 0; r < RS_R; r++) {
-    const uint32_t i = min(base + r * RS_T + tid, n - 1);
-    key[r] = D == 0 ? rs_key(pb[i]) : kin[i];
+    for (uint32_t r = 0; r < RS_R; r++) {
+      const uint32_t i = base + r * RS_T + tid;
+      p[r] = i < n ? pb[i] : 0.0f;
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < RS_R; r++) {
+      const uint32_t i = base + r * RS_T + tid;
+      p[r] *= inv;
+      key[r] = rs_key(p[r]);
+      if (i < n) pb[i] = p[r];
+    }
+    if (!sorts) return;
+  } else {
+#pragma unroll
+    for (uint32_t r = 0; r < RS_R; r++) key[r] = kin[min(base + r * RS_T + tid, n - 1)];
   }
   __syncthreads();
 #pragma unroll
   for (uint32_t r = 0; r < RS_R; r++)
     if (base + r * RS_T + tid < n) atomicAdd(&h[(key[r] >> (8 * D)) & 255u], 1u);
   __syncthreads();
-  cnt[tid * G + blockIdx.x] = h[tid];
+  cnt[G <= RS_SELF ? blockIdx.x * 256 + tid : tid * G + blockIdx.x] = h[tid];
 }
 
-// exclusive prefix sum of cnt[0..e) in place, one workgroup of CW threads.
-// With LDS (e <= RS_SCAN_LDS words) the counts are staged there by coalesced
-// loads, each thread scans a contiguous chunk, and the result goes back
-// coalesced; otherwise the chunks are read from global memory.
-constexpr uint32_t RS_SCAN_LDS = 32768;
-template <bool LDS>
+// exclusive prefix sum of cnt[0..e) in place, one workgroup of CW threads
 __global__ __launch_bounds__(CW) void k_rs_scan(uint32_t* cnt, uint32_t e, const cx_samp_state* sd) {
   if (sd->top_p >= 1.0f) return;
-  extern __shared__ uint32_t stage[];
   __shared__ uint32_t part[CW];
   const uint32_t tid = threadIdx.x, per = (e + CW - 1) / CW;
   const uint32_t lo = min(e, tid * per), hi = min(e, lo + per);
-  uint32_t* c = LDS ? stage : cnt;
-  if (LDS) {  // eight loads in flight a thread (a loop of one waited for each)
-    for (uint32_t i0 = tid; i0 < e; i0 += 8 * CW) {
-      uint32_t v[8];
-#pragma unroll
-      for (uint32_t u = 0; u < 8; u++) v[u] = cnt[min(i0 + u * CW, e - 1)];
-#pragma unroll
-      for (uint32_t u = 0; u < 8; u++)
-        if (i0 + u * CW < e) stage[i0 + u * CW] = v[u];
-    }
-    __syncthreads();
-  }
   uint32_t sum = 0;
-  for (uint32_t i = lo; i < hi; i++) sum += c[i];
+  for (uint32_t i = lo; i < hi; i++) sum += cnt[i];
   part[tid] = sum;
   __syncthreads();
   for (uint32_t off = 1; off < CW; off <<= 1) {  // inclusive scan of the parts
@@ -420,14 +417,40 @@ __global__ __launch_bounds__(CW) void k_rs_scan(uint32_t* cnt, uint32_t e, const
   }
   uint32_t run = part[tid] - sum;
   for (uint32_t i = lo; i < hi; i++) {
-    const uint32_t x = c[i];
-    c[i] = run;
+    const uint32_t x = cnt[i];
+    cnt[i] = run;
     run += x;
   }
-  if (LDS) {
-    __syncthreads();
-    for (uint32_t i = tid; i < e; i += CW) cnt[i] = stage[i];
+}
+
+// where digit `tid` of this tile starts, from the tile-major counts of the
+// G <= RS_SELF tiles: the digit's count in the tiles before, plus every
+// smaller digit's total
+__device__ inline uint32_t rs_offset(const uint32_t* cnt, uint32_t G) {
+  __shared__ uint32_t wsum[RS_T / 64];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  uint32_t before = 0, total = 0;
+  for (uint32_t t0 = 0; t0 < G; t0 += 16) {
+    uint32_t v[16];
+#pragma unroll
+    for (uint32_t u = 0; u < 16; u++) v[u] = cnt[min(t0 + u, G - 1) * 256 + tid];
+#pragma unroll
+    for (uint32_t u = 0; u < 16; u++) {
+      if (t0 + u < G) total += v[u];
+      if (t0 + u < blockIdx.x) before += v[u];
+    }
   }
+  uint32_t incl = total;
+#pragma unroll
+  for (uint32_t off = 1; off < 64; off <<= 1) {
+    const uint32_t v = __shfl_up(incl, off);
+    if (lane >= off) incl += v;
+  }
+  if (lane == 63) wsum[w] = incl;
+  __syncthreads();
+  uint32_t base = incl - total;
+  for (uint32_t v = 0; v < w; v++) base += wsum[v];
+  return base + before;
 }
 
 template <int D>
@@ -441,7 +464,7 @@ __global__ __launch_bounds__(RS_T) void k_rs_scatter(const float* pb, const uint
   __shared__ uint32_t wc[4][256];   // digit counts of each wave in this round
   const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6, base = blockIdx.x * RS_TILE;
   const uint64_t below = (1ull << lane) - 1;
-  run[tid] = off[tid * G + blockIdx.x];
+  run[tid] = G <= RS_SELF ? rs_offset(off, G) : off[tid * G + blockIdx.x];
   // every round's key and index loaded before the first round (an index
   // past n reads element n - 1, never used)
   uint32_t keys[RS_R], idxs[RS_R];
@@ -575,19 +598,16 @@ int cx_launch_sample(const float* logits, size_t n, cx_samp_state* sd, float* pb
   CX_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_samp_sum, dim3(1), dim3(CW), RING_LDS, s, pb, N, sd);
   CX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_samp_p, dim3(g), dim3(ZB), 0, s, pb, N, sd);
-  CX_HIP(hipGetLastError());
   // the descending order: pb -> (kA, iA) -> (kB, ord) -> (kA, iA) -> ord, ordp
   const uint32_t E = 256 * G;
   auto pass = [&](auto count, auto scatter, const uint32_t* ki, const uint32_t* ii, uint32_t* ko,
                   uint32_t* io, float* po) -> int {
     hipLaunchKernelGGL(count, dim3(G), dim3(RS_T), 0, s, pb, ki, N, sd, cnt, G);
     CX_HIP(hipGetLastError());
-    if (E <= RS_SCAN_LDS)
-      hipLaunchKernelGGL(k_rs_scan<true>, dim3(1), dim3(CW), E * 4, s, cnt, E, sd);
-    else
-      hipLaunchKernelGGL(k_rs_scan<false>, dim3(1), dim3(CW), 0, s, cnt, E, sd);
-    CX_HIP(hipGetLastError());
+    if (G > RS_SELF) {
+      hipLaunchKernelGGL(k_rs_scan, dim3(1), dim3(CW), 0, s, cnt, E, sd);
+      CX_HIP(hipGetLastError());
+    }
     hipLaunchKernelGGL(scatter, dim3(G), dim3(RS_T), 0, s, pb, ki, ii, N, sd, cnt, G, ko, io, po);
     CX_HIP(hipGetLastError());
     return CX_OK;

@@ -58,6 +58,17 @@ def test_sampler_matches_oracle(S, dev, kind, n, temp, top_p):
     assert g.estado == o.state
 
 
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 32768 + 1, 128 * 2048, 128 * 2048 + 1])
+def test_sort_tiles(S, dev, n):
+    """Around one tile of the sort (2048 tokens), the offsets' rounds of 16
+    tiles, and 128 tiles, above which the offsets come from a launch of their
+    own; ties at every level, so a wrong order shows."""
+    lg = logits_of("steps", n, n)
+    d = torch.from_numpy(lg).to(dev)
+    g, o = S.Muestreador(n, 1.0, 0.97), O.Sampler(n, 1.0, 0.97)
+    assert [g.elegir(d) for _ in range(6)] == [o.choose(lg) for _ in range(6)]
+
+
 def test_a_nan_top_p_keeps_the_candidates(S, dev):
     """top_p NaN (f32::clamp keeps it): the candidates' mass is not below it,
     so the nucleus is the 1024 most probable tokens, whole
