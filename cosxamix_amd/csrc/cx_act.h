@@ -200,10 +200,147 @@ __device__ inline double cx_rms_seq_sum(const float* x, uint32_t n) {
   return __shfl(s, 0, 64);
 }
 
+// The same sum by a 256-thread workgroup (n % 4 == 0, x 16-byte aligned, every
+// x finite), without one dependent add a value. A launch over
+// 512 rows lasts as long as its rows that take this sum: k_norm_quant_gemm
+// at k = 2048 17.7 -> 12.3 us, at 4096 35.9 -> 17.1 (5.3 where no row does).
+// What bounds it is the chain of its rounds, one for each binade.
+//
+// While the running sum s stays in one binade [2^E, 2^(E+1)), whose f64 values
+// are the multiples of u = 2^(E-52), what an add of t contributes depends on s
+// only where t lies halfway between multiples of u, and then only on the last
+// bit of s. So a thread's run of values acts on s as one of two additions, one
+// for each last bit: it adds its values to 2^E and to 2^E + u and keeps the two
+// differences and the two last bits. Such pairs compose, so a scan over the
+// threads gives each one's incoming sum. From the first thread whose sum
+// reaches 2^(E+1) on they don't hold: that thread adds its values to its
+// (exact) incoming sum, and the threads after it start again in the new
+// binade. (A run that leaves the binade from 2^E leaves it from any s there,
+// so it is seen; differences only grow, so a sum past the top stays past it.)
+// A sum that is still 0 takes 0 for both starts and stops at the first value.
+// The first CX_RMS_HEAD values, where the sum doubles every few threads, are
+// added by one wave.
+constexpr uint32_t CX_RMS_HEAD = 128;
+struct cx_rms_run {
+  double d0, d1;  // added to an s whose last bit is 0, 1
+  uint32_t q;     // bit p: the last bit after, from last bit p
+};
+__device__ inline cx_rms_run cx_rms_then(const cx_rms_run& f, const cx_rms_run& g) {
+  cx_rms_run r;
+  const uint32_t f0 = f.q & 1, f1 = (f.q >> 1) & 1;
+  r.d0 = f.d0 + (f0 ? g.d1 : g.d0);
+  r.d1 = f.d1 + (f1 ? g.d1 : g.d0);
+  r.q = ((g.q >> f0) & 1) | (((g.q >> f1) & 1) << 1);
+  return r;
+}
+// the run of the lane that DPP control CTRL names; the one that adds nothing
+// where it names none or the lane's row is not in ROWS
+template <int CTRL, int ROWS>
+__device__ inline double cx_dpp_d(double v) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xF, false);
+  const uint32_t hi =
+      (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xF, false);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+template <int CTRL, int ROWS>
+__device__ inline cx_rms_run cx_rms_from(const cx_rms_run& r) {
+  return cx_rms_run{cx_dpp_d<CTRL, ROWS>(r.d0), cx_dpp_d<CTRL, ROWS>(r.d1),
+                    (uint32_t)__builtin_amdgcn_update_dpp(2, (int)r.q, CTRL, ROWS, 0xF, false)};
+}
+__device__ inline double cx_rms_seq_sum_wg(const float* x, uint32_t n) {
+  __shared__ cx_rms_run wrun[4];  // the waves' runs
+  __shared__ double wsum[4];      // the sum after a wave's first thread that leaves the binade
+  __shared__ uint32_t wat[4];     // that thread, or 256
+  const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const uint32_t head = min(n, CX_RMS_HEAD);
+  if (tid < 64) {
+    const double h = cx_rms_seq_sum(x, head);
+    if (tid == 0) wsum[0] = h;
+  }
+  __syncthreads();
+  double s = wsum[0];
+  for (uint32_t b = head; b < n;) {
+    const uint32_t quads = min(4u, (n - b + 1023) / 1024);  // float4s a thread this time
+    double t[16];
+#pragma unroll
+    for (uint32_t g = 0; g < 4; g++) {
+      const uint32_t i = b + 4 * (tid * quads + g);
+      const float4 f = g < quads && i < n ? *reinterpret_cast<const float4*>(x + i)
+                                          : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      t[4 * g] = (double)f.x * (double)f.x;
+      t[4 * g + 1] = (double)f.y * (double)f.y;
+      t[4 * g + 2] = (double)f.z * (double)f.z;
+      t[4 * g + 3] = (double)f.w * (double)f.w;
+    }
+    for (uint32_t from = 0; from < 256;) {  // threads before `from` are done
+      const uint64_t e = (uint64_t)__double_as_longlong(s) & 0x7FF0000000000000ull;
+      const double lo = __longlong_as_double((long long)e);
+      const double lo1 = s > 0.0 ? __longlong_as_double((long long)(e | 1)) : 0.0;
+      const uint32_t p = (uint32_t)__double_as_longlong(s) & 1;
+      cx_rms_run r{0.0, 0.0, 2u};  // adds nothing
+      if (tid >= from) {
+        double a0 = lo, a1 = lo1;
+#pragma unroll
+        for (uint32_t g = 0; g < 4; g++)
+          if (g < quads) {
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++) {
+              a0 += t[4 * g + j];
+              a1 += t[4 * g + j];
+            }
+          }
+        r.d0 = a0 - lo;
+        r.d1 = a1 - lo1;
+        r.q = ((uint32_t)__double_as_longlong(a0) & 1) |
+              (((uint32_t)__double_as_longlong(a1) & 1) << 1);
+      }
+      // the scan over the lanes, in row shifts and row broadcasts (through
+      // ds_bpermute its six steps took most of the sum's time)
+      r = cx_rms_then(cx_rms_from<0x111, 0xF>(r), r);  // row_shr:1
+      r = cx_rms_then(cx_rms_from<0x112, 0xF>(r), r);  // row_shr:2
+      r = cx_rms_then(cx_rms_from<0x114, 0xF>(r), r);  // row_shr:4
+      r = cx_rms_then(cx_rms_from<0x118, 0xF>(r), r);  // row_shr:8
+      r = cx_rms_then(cx_rms_from<0x142, 0xA>(r), r);  // row_bcast:15 into rows 1, 3
+      r = cx_rms_then(cx_rms_from<0x143, 0xC>(r), r);  // row_bcast:31 into rows 2, 3
+      if (lane == 63) wrun[w] = r;
+      __syncthreads();
+      cx_rms_run f{0.0, 0.0, 2u};
+      for (uint32_t v = 0; v < w; v++) f = cx_rms_then(f, wrun[v]);
+      r = cx_rms_then(f, r);
+      const double after = s + (p ? r.d1 : r.d0), front = s + (p ? f.d1 : f.d0);
+      double before = cx_dpp_d<0x138, 0xF>(after);  // wave_shr:1
+      if (lane == 0) before = front;
+      // lo is 2^E, lo + lo its top; from 0 any value leaves
+      const uint64_t out = __ballot(s > 0.0 ? after >= lo + lo : after > 0.0);
+      const uint32_t at = out ? (uint32_t)__builtin_ctzll(out) : 63u;
+      if (lane == at) {
+        if (out) {
+          double a = before;
+#pragma unroll
+          for (uint32_t j = 0; j < 16; j++) a += t[j];  // (values past the run are +0.0)
+          wsum[w] = a;
+        } else {
+          wsum[w] = after;
+        }
+        wat[w] = out ? tid : 256u;
+      }
+      __syncthreads();
+      uint32_t c = 3;  // the first wave that leaves, or the last one
+      for (int v = 2; v >= 0; v--) c = wat[v] < 256 ? (uint32_t)v : c;
+      s = wsum[c];
+      from = wat[c] + 1;
+    }
+    b += 1024 * quads;
+  }
+  __syncthreads();  // wsum is free again
+  return s;
+}
+
 // The rmsnorm factor of x[0..n) (n % 4 == 0, x 16-byte aligned) over a
 // 256-thread workgroup, bit for bit the reference's: the tree (4 values a
 // lane, wave sums, ((w0 + w1) + w2) + w3), the check above, and the sum in
-// order when the check asks for it. `red` is 9 doubles and `flag` an int of
+// order when the check asks for it. `red` is 8 doubles and `flag` an int of
 // shared memory; every thread of the workgroup calls it.
 __device__ inline double cx_rms_scale(const float* x, uint32_t n, float eps, double* red,
                                       int* flag) {
@@ -237,12 +374,7 @@ __device__ inline double cx_rms_scale(const float* x, uint32_t n, float eps, dou
   if (reach && risk.unsure(reach)) *flag = 1;
   __syncthreads();
   if (*flag) {  // the same for every thread
-    if (tid < 64) {
-      const double seq = cx_rms_seq_sum(x, n);
-      if (tid == 0) red[8] = seq;
-    }
-    __syncthreads();
-    scale = cx_rms_factor(red[8], n, eps);
+    scale = cx_rms_factor(cx_rms_seq_sum_wg(x, n), n, eps);
   }
   __syncthreads();  // red and flag are free again
   return scale;

@@ -1098,7 +1098,7 @@ template <int SUB>
 __global__ __launch_bounds__(256) void k_norm_quant_gemm(const float* x, const float* w,
                                                          uint32_t m, uint32_t k, float eps,
                                                          uint32_t m_pad, int8_t* xq, float* xexs) {
-  __shared__ double red[9];
+  __shared__ double red[8];
   __shared__ int flag;
   const int tid = threadIdx.x;
   const uint32_t a = blockIdx.x;

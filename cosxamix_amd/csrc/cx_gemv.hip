@@ -2477,7 +2477,7 @@ __global__ __launch_bounds__(256) void k_swiglu_quant(const float* g, const floa
 template <int SUB>
 __global__ __launch_bounds__(256) void k_norm_quant(const float* x, const float* w, uint32_t n,
                                                     float eps, int8_t* xq, float* xe, float* xs) {
-  __shared__ double red[9];
+  __shared__ double red[8];
   __shared__ int flag;
   const double scale = cx_rms_scale(x, n, eps, red, &flag);
   for (uint32_t i = 8 * threadIdx.x; i < n; i += 8 * 256) {  // n % SUB == 0: whole groups
@@ -2496,7 +2496,7 @@ __global__ __launch_bounds__(256) void k_norm_quant(const float* x, const float*
 // batched prefill matches token-by-token decoding.
 __global__ __launch_bounds__(256) void k_norm_rows(const float* x, const float* w, uint32_t k,
                                                    float eps, float* out) {
-  __shared__ double red[9];
+  __shared__ double red[8];
   __shared__ int flag;
   const int tid = threadIdx.x;
   const float* xr = x + (size_t)blockIdx.x * k;
@@ -2540,7 +2540,7 @@ __global__ __launch_bounds__(256) void k_add_rows(float* y, const float* a, uint
 
 __global__ __launch_bounds__(256) void k_rmsnorm(float* out, const float* in, const float* w,
                                                  uint32_t n, float eps) {
-  __shared__ double red[9];
+  __shared__ double red[8];
   __shared__ int flag;
   const float* x = in + (size_t)blockIdx.x * n;
   float* y = out + (size_t)blockIdx.x * n;

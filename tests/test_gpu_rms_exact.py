@@ -22,12 +22,15 @@ from oracle import oracle as O
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [2048, 4096, 896, 1024])
+@pytest.mark.parametrize("n", [2048, 4096, 896, 1024, 160, 1152, 1184, 4224, 4256, 11008])
 def test_rmsnorm_operator_on_splitting_vectors(dev, n):
+    """The first four are the models' widths; the others lie around the
+    workgroup sum's head (128 values) and its passes of 1024 to 4096."""
     from cosxamix_amd import ops
     rows = []
     for seed in range(3):
-        x, j = R.splitting_vector(n, seed)
+        x, j = R.splitting_vector(n, seed, trees=("tree4",) if n not in (2048, 4096, 896, 1024)
+                                  else ("tree8", "tree4"))
         s = R.seq_sum(x)
         # the teeth: the operator's tree alone would give another f32 at j
         assert R.f32_of(x[j], R.factor(R.tree4_sum(x), n, 1e-6)) != R.f32_of(x[j], R.factor(s, n, 1e-6))
