@@ -62,13 +62,17 @@ cx_lib* cx_lib_get() {
   if (!L) {
     if (hipSetDevice(dev) != hipSuccess) return nullptr;
     hipStream_t s = nullptr;
-    hipEvent_t ev = nullptr;
+    hipEvent_t ev[2] = {nullptr, nullptr};
     if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return nullptr;
-    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+    if (hipEventCreateWithFlags(&ev[0], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&ev[1], hipEventDisableTiming) != hipSuccess) {
+      if (ev[0]) (void)hipEventDestroy(ev[0]);
       (void)hipStreamDestroy(s);
       return nullptr;
     }
-    L = new cx_lib{dev, s, nullptr, 0, ev, false};
+    L = new cx_lib{dev, s, {}, {}};
+    L->scratch.used = ev[0];
+    L->att.used = ev[1];
   }
   t_ctx.ctx[dev] = L;
   return L;
@@ -79,8 +83,8 @@ static bool capturing(hipStream_t s) {
   return hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
-// The calling thread's scratch of at least `bytes`, for work about to be
-// enqueued on stream s. s first waits for the `used` event, which follows
+// The calling thread's scratch (or its other buffer) of at least `bytes`, for
+// work about to be enqueued on stream s. s first waits for the `used` event, which follows
 // every earlier use of the scratch on any stream (each use waited for the
 // one before it), by this thread or by the thread that held the context
 // before. Growing frees the old buffer and allocates the new one in s's
@@ -88,41 +92,43 @@ static bool capturing(hipStream_t s) {
 // or thread is waited for. Under stream capture the scratch cannot grow and
 // the captured work is not ordered after earlier uses: the caller orders its
 // graph's launches, as for any captured work.
-int cx_scratch_acquire(size_t bytes, hipStream_t s, void** out) {
+int cx_scratch_acquire(cx_buffer cx_lib::*which, size_t bytes, hipStream_t s, void** out) {
   cx_lib* L = cx_lib_get();
   if (!L) {
     cx_set_error("no HIP device %d", g_device);
     return CX_EHIP;
   }
+  cx_buffer& B = L->*which;
   const bool cap = capturing(s);
-  if (!cap && L->used_valid) CX_HIP(hipStreamWaitEvent(s, L->used, 0));
-  if (L->scratch_bytes < bytes) {
+  if (!cap && B.used_valid) CX_HIP(hipStreamWaitEvent(s, B.used, 0));
+  if (B.bytes < bytes) {
     CX_REQUIRE(!cap,
                "the calling thread's scratch must grow to %zu bytes while the stream is being "
                "captured: make the same call once before the capture, or use "
                "cx_matmul_auto_noalloc",
                bytes);
     CX_HIP(hipSetDevice(L->device));
-    if (L->scratch) CX_HIP(hipFreeAsync(L->scratch, s));
-    L->scratch = nullptr;
-    L->scratch_bytes = 0;
-    CX_HIP(hipMallocAsync(&L->scratch, bytes, s));
-    L->scratch_bytes = bytes;
+    if (B.p) CX_HIP(hipFreeAsync(B.p, s));
+    B.p = nullptr;
+    B.bytes = 0;
+    CX_HIP(hipMallocAsync(&B.p, bytes, s));
+    B.bytes = bytes;
   }
-  *out = L->scratch;
+  *out = B.p;
   return CX_OK;
 }
 
-void cx_scratch_release(hipStream_t s) {
+void cx_scratch_release(cx_buffer cx_lib::*which, hipStream_t s) {
   cx_lib* L = cx_lib_get();
   if (!L || capturing(s)) return;
-  if (hipEventRecord(L->used, s) == hipSuccess) {
-    L->used_valid = true;
+  cx_buffer& B = L->*which;
+  if (hipEventRecord(B.used, s) == hipSuccess) {
+    B.used_valid = true;
     return;
   }
   // without the event the next use could not be ordered: finish the work
   (void)hipStreamSynchronize(s);
-  L->used_valid = false;
+  B.used_valid = false;
 }
 
 static int noalloc_scratch(int dev, void** out);
@@ -521,9 +527,9 @@ extern "C" int cx_attention(const float* q, const float* k, const float* v, size
   CX_REQUIRE(q && k && v && out, "attention: null pointer");
   hipStream_t s = STREAM(stream);
   // Many query tokens on the kernels made for them, in slabs of tokens whose
-  // scores fit kAttnSlabBytes of the thread's scratch. A captured call keeps to
-  // the general kernel, which needs no scratch: a graph must not hold a
-  // buffer that a later call may replace.
+  // scores fit kAttnSlabBytes of the thread's buffer for them. A captured call
+  // keeps to the general kernel, which needs no buffer: a graph must not hold
+  // one that a later call may replace.
   const bool many = kv_heads && heads >= kv_heads && heads % kv_heads == 0 && tokens > 0 &&
                     tokens <= total && total <= CX_ATT_MAX_TOTAL && heads <= 128 &&
                     cx_attn_many_suits_general(tokens, total, heads, hd) &&
@@ -536,7 +542,7 @@ extern "C" int cx_attention(const float* q, const float* k, const float* v, size
   slab = tokens < slab ? tokens : slab < 64 ? 64 : slab;
   const cx_attn_many_floats f = cx_attn_many_scratch(slab, total, heads, kv_heads);
   void* sp = nullptr;
-  cx_scratch scr(s);
+  cx_scratch scr(s, &cx_lib::att);
   int rc = scr.get(up(f.sc) + up(f.cm) + up(f.inv), &sp);
   if (rc) {  // no room for the scores: the general kernel needs none
     (void)hipGetLastError();

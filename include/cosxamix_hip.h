@@ -27,12 +27,13 @@
  *     once (src/ops.rs:487-500): each host thread has its own stream and
  *     device scratch. Level-2 functions may run on several threads at once.
  *     The calls that use a thread's scratch (cx_matmul_auto,
- *     cx_matmul_multi_1row, cx_gemv_subsums, cx_dequantize_rows, cx_attention
- *     (outside a capture), cx_attention_decode, cx_sample) are ordered on the device after that
+ *     cx_matmul_multi_1row, cx_gemv_subsums, cx_dequantize_rows,
+ *     cx_attention_decode, cx_sample) are ordered on the device after that
  *     scratch's previous use, whatever stream it was on, also when a thread
  *     ends with work still queued and another thread takes its scratch; the
  *     host is not blocked, and a growing scratch is reallocated in stream
- *     order. Under stream capture the scratch cannot grow (CX_EINVAL: make
+ *     order. cx_attention's larger calls are ordered among themselves in the
+ *     same way, by a buffer that no other call uses. Under stream capture the scratch cannot grow (CX_EINVAL: make
  *     the call once before capturing) and the caller orders the graph's
  *     launches. A cx_model and its caches are used by one thread at a time;
  *     the reference serialises generation behind a Mutex
@@ -210,8 +211,8 @@ int cx_softmax(float *x, size_t len, size_t width, void *stream);
 
 /* ops::atencion (src/ops.rs:1258-1325): causal GQA. q[tokens][H*hd],
  * k/v[total][Hkv*hd], out[tokens][H*hd]. In the reference's order. Larger
- * calls keep their scores in the thread's scratch (up to 256 MB); a captured
- * call uses none. */
+ * calls keep their scores in a buffer of the thread's (up to 256 MB) that no
+ * other call uses and no graph holds; a captured call uses none. */
 int cx_attention(const float *q, const float *k, const float *v, size_t tokens,
                  size_t total, size_t heads, size_t kv_heads, size_t head_dim,
                  float *out, void *stream);

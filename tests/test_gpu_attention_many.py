@@ -94,3 +94,32 @@ def test_capture_and_misaligned_rows_take_the_general_kernel(dev):
     out.fill_(7.0)
     ops.atencion(flat[1:].reshape(q.shape), kd, vd, forma, out)  # 4-byte aligned
     assert same(out.cpu().numpy(), want)
+
+
+def test_attention_leaves_a_captured_graphs_scratch_alone(dev):
+    # a graph holds the address of the scratch it was captured with: attention
+    # between its replays neither grows that scratch nor writes to it
+    from cosxamix_amd import ops
+    m, n, k = 8, 64, 256
+    w = torch.from_numpy(O.daiss_matrix(3, "w", n, k, 0.02, O.Q4_K)).to(dev)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(1)).to(dev)
+    y = torch.zeros(m, n, device=dev)
+    ops.matmul_auto((m, k, n), x, w, O.Q4_K, y)  # the scratch has its size
+    want = y.clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ops.matmul_auto((m, k, n), x, w, O.Q4_K, y)
+    q, kk, v = inputs(4, 300, 2000, 16, 2, 128)  # ~37 MB of scores
+    qd, kd, vd = (torch.from_numpy(t).to(dev) for t in (q, kk, v))
+    first, again = torch.zeros_like(qd), torch.zeros_like(qd)
+    side = torch.cuda.Stream()
+    ops.atencion(qd, kd, vd, (300, 2000, 16, 2, 128), first)
+    for _ in range(4):
+        y.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):  # beside the graph
+            ops.atencion(qd, kd, vd, (300, 2000, 16, 2, 128), again)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int32), want.view(torch.int32))
+        assert torch.equal(again.view(torch.int32), first.view(torch.int32))
