@@ -83,6 +83,14 @@ static bool capturing(hipStream_t s) {
   return hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
+// Whether work on stream s runs on the device of the calling thread's context,
+// where its buffers are (cx_init; a call may come with another device's stream)
+static bool on_thread_device(hipStream_t s) {
+  int dev = -1;
+  const hipError_t e = s ? hipStreamGetDevice(s, &dev) : hipGetDevice(&dev);
+  return e == hipSuccess && dev == g_device;
+}
+
 // The calling thread's scratch (or its other buffer) of at least `bytes`, for
 // work about to be enqueued on stream s. s first waits for the `used` event, which follows
 // every earlier use of the scratch on any stream (each use waited for the
@@ -529,11 +537,13 @@ extern "C" int cx_attention(const float* q, const float* k, const float* v, size
   // Many query tokens on the kernels made for them, in slabs of tokens whose
   // scores fit kAttnSlabBytes of the thread's buffer for them. A captured call
   // keeps to the general kernel, which needs no buffer: a graph must not hold
-  // one that a later call may replace.
+  // one that a later call may replace. So does a call on another device than the
+  // thread's, whose buffer is not there.
   const bool many = kv_heads && heads >= kv_heads && heads % kv_heads == 0 && tokens > 0 &&
                     tokens <= total && total <= CX_ATT_MAX_TOTAL && heads <= 128 &&
                     cx_attn_many_suits_general(tokens, total, heads, hd) &&
-                    (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0 && !capturing(s);
+                    (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0 && !capturing(s) &&
+                    on_thread_device(s);
   if (!many) return cx_launch_attention(q, k, v, tokens, total, heads, kv_heads, hd, out, s);
   const cx_attn_many_floats s64 = cx_attn_many_scratch(64, total, heads, kv_heads);
   auto up = [](size_t floats) { return (floats * 4 + 255) / 256 * 256; };

@@ -123,3 +123,17 @@ def test_attention_leaves_a_captured_graphs_scratch_alone(dev):
         torch.cuda.synchronize()
         assert torch.equal(y.view(torch.int32), want.view(torch.int32))
         assert torch.equal(again.view(torch.int32), first.view(torch.int32))
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs a second GPU")
+def test_another_devices_stream_takes_the_general_kernel(dev):
+    # the thread's context is on device 0; the call's tensors and stream on 1
+    from cosxamix_amd import ops
+    tokens, total, heads, kv, hd = 70, 1040, 4, 2, 64
+    q, k, v = inputs(3, tokens, total, heads, kv, hd)
+    with torch.cuda.device(1):
+        out = torch.full(q.shape, 7.0, dtype=torch.float32, device="cuda:1")
+        ops.atencion(*(torch.from_numpy(t).to("cuda:1") for t in (q, k, v)),
+                     (tokens, total, heads, kv, hd), out)
+        assert torch.cuda.current_device() == 1
+        assert same(out.cpu().numpy(), oracle(q, k, v, heads, kv, hd))
