@@ -542,8 +542,8 @@ extern "C" int cx_attention(const float* q, const float* k, const float* v, size
   const bool many = kv_heads && heads >= kv_heads && heads % kv_heads == 0 && tokens > 0 &&
                     tokens <= total && total <= CX_ATT_MAX_TOTAL && heads <= 128 &&
                     cx_attn_many_suits_general(tokens, total, heads, hd) &&
-                    (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0 && !capturing(s) &&
-                    on_thread_device(s);
+                    (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) == 0 &&
+                    !capturing(s) && on_thread_device(s);
   if (!many) return cx_launch_attention(q, k, v, tokens, total, heads, kv_heads, hd, out, s);
   const cx_attn_many_floats s64 = cx_attn_many_scratch(64, total, heads, kv_heads);
   auto up = [](size_t floats) { return (floats * 4 + 255) / 256 * 256; };

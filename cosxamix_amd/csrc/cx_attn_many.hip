@@ -500,7 +500,7 @@ int cx_launch_attn_many(const cx_attn_many_args& a, hipStream_t s) {
   CX_REQUIRE(a.hd == 64 || a.hd == 128, "attention: head_dim %u (64 or 128 supported)", a.hd);
   CX_REQUIRE(a.kvh && a.heads % a.kvh == 0, "attention: %u heads / %u groups", a.heads, a.kvh);
   CX_REQUIRE(a.tokens && a.sc && a.cm && a.inv, "attention: many query tokens need their scratch");
-  CX_REQUIRE((((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) & 15) == 0,
+  CX_REQUIRE((((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.out) & 15) == 0,
              "attention: rows must be 16-byte aligned");
   CX_REQUIRE((size_t)a.tokens * a.heads < (1u << 31) && (size_t)a.pos + a.tokens < (1u << 31),
              "attention: %u query tokens", a.tokens);

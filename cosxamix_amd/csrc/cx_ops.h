@@ -99,7 +99,7 @@ int cx_launch_att_scores(const cx_attn_args& a, float scale, hipStream_t s);
 // them), q and out rows of heads*hd; sc, cm and inv are scratch of at least
 // cx_attn_many_scratch(tokens, pos + tokens, heads, kvh) floats. Order-exact.
 struct cx_attn_many_args {
-  const float *q, *k, *v;  // 16-byte aligned
+  const float *q, *k, *v;  // 16-byte aligned, as out
   uint32_t tokens, pos, heads, kvh, hd;
   float *sc, *cm, *inv;
   float* out;

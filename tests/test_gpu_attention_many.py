@@ -96,6 +96,25 @@ def test_capture_and_misaligned_rows_take_the_general_kernel(dev):
     assert same(out.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("which", ["k", "v", "out"])
+def test_a_misaligned_tensor_takes_the_general_kernel(dev, which):
+    # the kernels of many tokens read q, k and v and write out 16 bytes at a
+    # time; a view at any float is an operand like any other
+    from cosxamix_amd import ops
+    tokens, total, heads, kv, hd = 70, 1040, 4, 2, 64
+    q, k, v = inputs(3, tokens, total, heads, kv, hd)
+    t = dict(q=torch.from_numpy(q).to(dev), k=torch.from_numpy(k).to(dev),
+             v=torch.from_numpy(v).to(dev), out=torch.full(q.shape, 7.0, device=dev))
+    flat = torch.full((t[which].numel() + 8,), 7.0, device=dev)
+    flat[1:1 + t[which].numel()] = t[which].reshape(-1)
+    t[which] = flat[1:1 + t[which].numel()].reshape(t[which].shape)
+    assert t[which].data_ptr() % 16 == 4
+    ops.atencion(t["q"], t["k"], t["v"], (tokens, total, heads, kv, hd), t["out"])
+    assert same(t["out"].cpu().numpy(), oracle(q, k, v, heads, kv, hd))
+    if which == "out":  # nothing beside it written
+        assert torch.all(flat[:1] == 7.0) and torch.all(flat[1 + q.size:] == 7.0)
+
+
 def test_attention_leaves_a_captured_graphs_scratch_alone(dev):
     # a graph holds the address of the scratch it was captured with: attention
     # between its replays neither grows that scratch nor writes to it
