@@ -524,18 +524,13 @@ extern "C" int cx_softmax(float* x, size_t len, size_t width, void* stream) {
   return cx_launch_softmax(x, len, width, STREAM(stream));
 }
 
-// the scores of one slab of query tokens in cx_attention; the largest calls take
-// a few slabs (a slab of 64 tokens at least: 131 MB at 32 heads and 16000
-// positions)
-static const size_t kAttnSlabBytes = 256ull << 20;
-
 extern "C" int cx_attention(const float* q, const float* k, const float* v, size_t tokens,
                             size_t total, size_t heads, size_t kv_heads, size_t hd, float* out,
                             void* stream) {
   CX_REQUIRE(q && k && v && out, "attention: null pointer");
   hipStream_t s = STREAM(stream);
   // Many query tokens on the kernels made for them, in slabs of tokens whose
-  // scores fit kAttnSlabBytes of the thread's buffer for them. A captured call
+  // scores fit the thread's buffer for them (cx_attn_many_slab). A captured call
   // keeps to the general kernel, which needs no buffer: a graph must not hold
   // one that a later call may replace. So does a call on another device than the
   // thread's, whose buffer is not there.
@@ -545,11 +540,8 @@ extern "C" int cx_attention(const float* q, const float* k, const float* v, size
                     (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) == 0 &&
                     !capturing(s) && on_thread_device(s);
   if (!many) return cx_launch_attention(q, k, v, tokens, total, heads, kv_heads, hd, out, s);
-  const cx_attn_many_floats s64 = cx_attn_many_scratch(64, total, heads, kv_heads);
   auto up = [](size_t floats) { return (floats * 4 + 255) / 256 * 256; };
-  // 64 tokens are whole tiles of rows whatever the heads per group
-  size_t slab = kAttnSlabBytes / ((s64.sc + s64.cm + s64.inv) * 4) * 64;
-  slab = tokens < slab ? tokens : slab < 64 ? 64 : slab;
+  const size_t slab = cx_attn_many_slab(tokens, total, heads, kv_heads);
   const cx_attn_many_floats f = cx_attn_many_scratch(slab, total, heads, kv_heads);
   void* sp = nullptr;
   cx_scratch scr(s, &cx_lib::att);

@@ -496,6 +496,25 @@ cx_attn_many_floats cx_attn_many_scratch(size_t tokens, size_t total, size_t hea
   return {rows * total, rows * ((total + MQ_C - 1) / MQ_C), rows};
 }
 
+// 256 MB: 256 tokens at 32 heads and 8000 positions, so that only the largest
+// calls take several slabs. 64 tokens are whole tiles of rows whatever the heads
+// a group; where they alone are more (128 heads, 8192 positions), as few as fill
+// one 64-row tile a group.
+size_t cx_attn_many_slab(size_t tokens, size_t total, size_t heads, size_t kvh) {
+  constexpr size_t budget = 256ull << 20;
+  auto bytes = [&](size_t t) {
+    const cx_attn_many_floats f = cx_attn_many_scratch(t, total, heads, kvh);
+    return (f.sc + f.cm + f.inv) * 4;
+  };
+  if (bytes(tokens) <= budget) return tokens;
+  size_t slab = 64;
+  if (bytes(64) <= budget)
+    slab = budget / bytes(64) * 64;
+  else
+    while (bytes(slab) > budget && slab * (heads / kvh) > MQ_R) slab /= 2;
+  return slab < tokens ? slab : tokens;
+}
+
 int cx_launch_attn_many(const cx_attn_many_args& a, hipStream_t s) {
   CX_REQUIRE(a.hd == 64 || a.hd == 128, "attention: head_dim %u (64 or 128 supported)", a.hd);
   CX_REQUIRE(a.kvh && a.heads % a.kvh == 0, "attention: %u heads / %u groups", a.heads, a.kvh);

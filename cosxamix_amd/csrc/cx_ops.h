@@ -113,6 +113,9 @@ struct cx_attn_many_floats {
 bool cx_attn_many_suits_prefill(size_t tokens, size_t total, size_t heads, size_t hd);
 bool cx_attn_many_suits_general(size_t tokens, size_t total, size_t heads, size_t hd);
 cx_attn_many_floats cx_attn_many_scratch(size_t tokens, size_t total, size_t heads, size_t kvh);
+// How many of `tokens` to take at a time: the scratch of as many is at most 256
+// MB, or what one 64-row tile of each KV group takes where that is more
+size_t cx_attn_many_slab(size_t tokens, size_t total, size_t heads, size_t kvh);
 int cx_launch_attn_many(const cx_attn_many_args& a, hipStream_t s);
 int cx_launch_attention(const float* q, const float* k, const float* v, size_t tokens,
                         size_t total, size_t heads, size_t kvh, size_t hd, float* out,

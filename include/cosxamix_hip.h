@@ -211,8 +211,10 @@ int cx_softmax(float *x, size_t len, size_t width, void *stream);
 
 /* ops::atencion (src/ops.rs:1258-1325): causal GQA. q[tokens][H*hd],
  * k/v[total][Hkv*hd], out[tokens][H*hd]. In the reference's order. Larger
- * calls keep their scores in a buffer of the thread's (up to 256 MB) that no
- * other call uses and no graph holds; a captured call uses none. */
+ * calls keep their scores in a buffer of the thread's that no other call uses
+ * and no graph holds: up to 256 MB, or about 260 * kv_heads * total bytes
+ * where that is more (533 MB at 128 KV heads and 16000 positions), held by the
+ * thread's context from then on. A captured call uses none. */
 int cx_attention(const float *q, const float *k, const float *v, size_t tokens,
                  size_t total, size_t heads, size_t kv_heads, size_t head_dim,
                  float *out, void *stream);

@@ -1,5 +1,6 @@
 """The host side of the attention of many query tokens (cx_attn_many.hip), without
-a GPU: what its launch refuses before any kernel runs."""
+a GPU: what its launch refuses before any kernel runs, and how many tokens
+cx_attention takes at a time for the memory it states."""
 import ctypes as C
 import re
 import subprocess
@@ -39,3 +40,34 @@ def test_a_misaligned_tensor_is_refused_before_any_launch(L, which):
     setattr(a, which, getattr(a, which) + 4)
     assert launch(C.byref(a), None) == L.CX_EINVAL
     assert b"aligned" in L.load().cx_last_error()
+
+
+class Floats(C.Structure):  # cx_attn_many_floats
+    _fields_ = [(n, C.c_size_t) for n in ("sc", "cm", "inv")]
+
+
+def test_a_slabs_scores_fit_the_memory_that_the_header_states(L):
+    slab, scratch = internal(L, "cx_attn_many_slab"), internal(L, "cx_attn_many_scratch")
+    slab.restype, slab.argtypes = C.c_size_t, [C.c_size_t] * 4
+    scratch.restype, scratch.argtypes = Floats, [C.c_size_t] * 4
+
+    def need(tokens, total, heads, kv):
+        f = scratch(tokens, total, heads, kv)
+        return (f.sc + f.cm + f.inv) * 4
+
+    for heads, kv in ((1, 1), (7, 1), (14, 2), (16, 2), (32, 8), (64, 64), (128, 1), (128, 8),
+                      (96, 32), (128, 128)):
+        for total in (64, 1000, 1024, 2048, 4097, 8192, 12000, 16000):
+            for tokens in (1, 2, 33, 63, 64, 65, 300, 512, 1999, total):
+                if tokens > total:
+                    continue
+                n = slab(tokens, total, heads, kv)
+                got = need(n, total, heads, kv)
+                assert 1 <= n <= tokens
+                assert got <= max(256 << 20, 260 * kv * total + 512 * kv), (tokens, total, heads, kv)
+                # no smaller than it has to be: all the tokens where they fit, else
+                # more than half of what would
+                if need(tokens, total, heads, kv) <= 256 << 20:
+                    assert n == tokens
+                elif need(2 * n, total, heads, kv) <= 256 << 20:
+                    assert 2 * n > tokens, (tokens, total, heads, kv, n)

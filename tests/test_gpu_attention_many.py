@@ -4,11 +4,14 @@ its tiles: rows (tokens x heads per group) around 64 and 128, positions around 3
 64 and 128, one to sixteen heads per group, both head dims, and every row count a
 lane takes. Values that a row does not see may be anything; a captured call and
 misaligned rows take the general kernel."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 from oracle import oracle as O
+from test_attention_many_plan import internal
 
 pytestmark = pytest.mark.gpu
 
@@ -54,6 +57,26 @@ def test_large_tiles_bit_exact(dev):
     q, k, v = inputs(5, tokens, total, heads, kv, hd)
     got = run(dev, q, k, v, heads, kv, hd)
     for t in (0, 1, 31, 32, 300, 510, 511):
+        n = total - tokens + t + 1
+        assert same(got[t], oracle(q[t:t + 1], k[:n], v[:n], heads, kv, hd)), t
+
+
+# Calls whose scores are more than the buffer holds (256 MB): tokens a slab, by
+# cx_attn_many_slab. The first and last tokens of every slab against the oracle.
+@pytest.mark.parametrize("tokens,total,heads,kv,hd,slab", [
+    (512, 8192, 32, 8, 128, 192),  # three slabs, the last of 128
+    (700, 12000, 14, 2, 64, 384),  # two
+    (70, 16000, 128, 8, 64, 32),   # below 64 tokens a slab; the last of 6
+    (3, 9000, 128, 128, 64, 3)])   # one tile of each group alone is more: all at once
+def test_slabs_bit_exact(dev, tokens, total, heads, kv, hd, slab):
+    from cosxamix_amd import _lib as L
+    plan = internal(L, "cx_attn_many_slab")
+    plan.restype, plan.argtypes = C.c_size_t, [C.c_size_t] * 4
+    assert plan(tokens, total, heads, kv) == slab
+    q, k, v = inputs(tokens + total, tokens, total, heads, kv, hd)
+    got = run(dev, q, k, v, heads, kv, hd)
+    edges = {t + d for t in range(0, tokens + 1, slab) for d in (-1, 0)} | {tokens - 1}
+    for t in sorted(e for e in edges if 0 <= e < tokens):
         n = total - tokens + t + 1
         assert same(got[t], oracle(q[t:t + 1], k[:n], v[:n], heads, kv, hd)), t
 
