@@ -1578,28 +1578,52 @@ static int run_steps(cx_cache* C, size_t prompt_end, size_t steps, float* step_m
 static const size_t kPrefillMaxT = 512;
 static const size_t kPrefillAttnBytes = 640ull << 20;  // attention scratch bound: 512 tokens at
                                                        // 32 heads up to 10000 positions
+// the second try, where memory is short
+static const size_t kPrefillShortT = 256;
+static const size_t kPrefillShortBytes = 256ull << 20;
+
+// Tokens a chunk (at most max_t) and the floats of its attention scratch over a
+// cache of cap positions, within attn_bytes or 16 tokens' worth where that is
+// more. The many-token kernels' part (rows in whole tiles of 64 a KV group) is
+// counted only for chunks long enough to take them; a chunk gives up tokens for
+// it down to 64 (whole tiles whatever the heads a group). inv 0: no chunk of this
+// cache takes those kernels.
+struct cx_prefill_size {
+  size_t T, sc, cm, inv;
+};
+cx_prefill_size cx_prefill_plan(size_t heads, size_t kvh, size_t hd, size_t cap, size_t max_t,
+                                size_t attn_bytes) {
+  const size_t sc = cx_attn_score_floats(heads, cap), cm = cx_attn_chunk_floats(heads, cap);
+  size_t T = attn_bytes / ((sc + cm) * 4);
+  T = T > max_t ? max_t : T < 16 ? 16 : T / 16 * 16;
+  if (T > cap) T = cap;
+  const cx_prefill_size few{T, T * sc, T * cm, 0};
+  // (fewer tokens or positions never make a chunk suited)
+  while (cx_attn_many_suits_prefill(T, cap, heads, hd)) {
+    const cx_attn_many_floats f = cx_attn_many_scratch(T, cap, heads, kvh);
+    const cx_prefill_size z{T, f.sc > T * sc ? f.sc : T * sc, f.cm > T * cm ? f.cm : T * cm, f.inv};
+    if ((z.sc + z.cm) * 4 <= attn_bytes) return z;
+    if (T <= 64) break;
+    T -= T % 16 ? T % 16 : 16;
+  }
+  return few;
+}
 
 static int prefill_alloc_chunk(cx_cache* C, size_t max_t, size_t attn_bytes) {
   cx_prefill& P = C->pf;
   const cx_config& c = C->m->cfg;
-  const size_t D = c.dim, hd = D / c.heads, kvd = c.kv_heads * hd, I = c.ffn, H = c.heads;
-  const size_t per_tok = (cx_attn_score_floats(H, C->cap) + cx_attn_chunk_floats(H, C->cap)) * 4;
-  size_t T = attn_bytes / per_tok;
-  T = T > max_t ? max_t : T < 16 ? 16 : T / 16 * 16;
-  if (T > C->cap) T = C->cap;
-  const size_t wide = D > I ? D : I;
-  // the scratch of either attention (few and many query tokens)
-  const cx_attn_many_floats f = cx_attn_many_scratch(T, C->cap, H, c.kv_heads);
-  const size_t sc = T * cx_attn_score_floats(H, C->cap), cm = T * cx_attn_chunk_floats(H, C->cap);
+  const size_t D = c.dim, hd = D / c.heads, kvd = c.kv_heads * hd, I = c.ffn;
+  const cx_prefill_size z = cx_prefill_plan(c.heads, c.kv_heads, hd, C->cap, max_t, attn_bytes);
+  const size_t T = z.T, wide = D > I ? D : I;
   struct Want {
     float** p;
     size_t floats;
   } want[] = {{&P.x, T * D},   {&P.nrm, T * wide}, {&P.q, T * D}, {&P.k, T * kvd},
               {&P.v, T * kvd}, {&P.att, T * D},    {&P.g, T * I}, {&P.u, T * I},
-              {&P.tmp, T * D}, {&P.sc, f.sc > sc ? f.sc : sc},    {&P.cm, f.cm > cm ? f.cm : cm},
-              {&P.inv, f.inv}};
+              {&P.tmp, T * D}, {&P.sc, z.sc},      {&P.cm, z.cm}, {&P.inv, z.inv}};
   bool ok = true;
-  for (const Want& w : want) ok = ok && hipMalloc(w.p, w.floats * 4) == hipSuccess;
+  for (const Want& w : want)
+    ok = ok && (!w.floats || hipMalloc(w.p, w.floats * 4) == hipSuccess);
   ok = ok && hipMalloc(&P.scratch, cx_gemm_scratch_bytes(T, wide)) == hipSuccess;
   if (ok) {
     P.T = (uint32_t)T;
@@ -1618,7 +1642,7 @@ static int prefill_alloc_chunk(cx_cache* C, size_t max_t, size_t attn_bytes) {
 static int prefill_alloc(cx_cache* C) {
   if (C->pf.T) return CX_OK;
   const int rc = prefill_alloc_chunk(C, kPrefillMaxT, kPrefillAttnBytes);
-  return rc ? prefill_alloc_chunk(C, kPrefillMaxT / 2, kPrefillAttnBytes / 4) : rc;
+  return rc ? prefill_alloc_chunk(C, kPrefillShortT, kPrefillShortBytes) : rc;
 }
 
 // out[r] = W . in[r] for `rows` rows of width k: the MFMA contraction,
@@ -1724,7 +1748,7 @@ static int enqueue_prefill_chunk(cx_cache* C, uint32_t pos, uint32_t nt) {
     if ((rc = cx_launch_rope_kv(P.q, P.k, P.v, kc, vc, m->cos_t, m->sin_t, c.heads, c.kv_heads,
                                 hd, C->st, nt, s)))
       return rc;
-    if (cx_attn_many_suits_prefill(nt, pos + nt, c.heads, hd)) {
+    if (P.inv && cx_attn_many_suits_prefill(nt, pos + nt, c.heads, hd)) {
       cx_attn_many_args a{};
       a.q = P.q;
       a.k = kc;

@@ -349,7 +349,11 @@ size_t cx_model_weight_bytes(const cx_model *m);
 /* forward::Cache (src/forward.rs:62-137), with room for `cap` tokens. A
  * cache belongs to its model: cx_model_free on a model with live caches
  * releases the model when its last cache is freed (caches can be freed
- * before or after their model). */
+ * before or after their model). Its first prefill (cx_forward or cx_generate
+ * over several tokens) allocates buffers for a chunk of up to 512 tokens, held
+ * until the cache is freed: every activation of the chunk and up to 640 MB of
+ * attention scores; where that much is not free, a chunk of up to 256 tokens
+ * and up to 256 MB (16 tokens' scores at least). */
 int cx_cache_new(cx_model *m, size_t cap, cx_cache **out);
 size_t cx_cache_len(const cx_cache *c);
 int cx_cache_truncate(cx_cache *c, size_t n);
