@@ -99,7 +99,8 @@ __device__ inline float cx_swiglu(float g, float u) {
 // moves v = x * scale by a bounded number of its ulps (cx_rms_reach). Where
 // no value's f32 rounding can change within that (cx_rms_risk), the tree's
 // scale gives the reference's outputs bit for bit;
-// otherwise the workgroup sums the squares again in order (cx_rms_seq_sum).
+// otherwise the workgroup sums the squares again in order (cx_rms_seq_sum, over
+// longer rows cx_rms_seq_sum_wg).
 // About one random vector in 300 takes the second sum at n = 2048, one in
 // 80 at n = 4096.
 // A lane's share of the tree: its sum of squares s, and w >= the share of
@@ -262,18 +263,22 @@ __device__ inline double cx_rms_seq_sum_wg(const float* x, uint32_t n) {
   double s = wsum[0];
   for (uint32_t b = head; b < n;) {
     const uint32_t quads = min(4u, (n - b + 1023) / 1024);  // float4s a thread this time
-    double t[16];
+    float t[16];
 #pragma unroll
     for (uint32_t g = 0; g < 4; g++) {
       const uint32_t i = b + 4 * (tid * quads + g);
       const float4 f = g < quads && i < n ? *reinterpret_cast<const float4*>(x + i)
                                           : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      t[4 * g] = (double)f.x * (double)f.x;
-      t[4 * g + 1] = (double)f.y * (double)f.y;
-      t[4 * g + 2] = (double)f.z * (double)f.z;
-      t[4 * g + 3] = (double)f.w * (double)f.w;
+      t[4 * g] = f.x;
+      t[4 * g + 1] = f.y;
+      t[4 * g + 2] = f.z;
+      t[4 * g + 3] = f.w;
     }
     for (uint32_t from = 0; from < 256;) {  // threads before `from` are done
+      // (opaque: squares kept over the rounds are 32 registers and, over many
+      // rows, half the waves a SIMD)
+#pragma unroll
+      for (uint32_t j = 0; j < 16; j++) asm volatile("" : "+v"(t[j]));
       const uint64_t e = (uint64_t)__double_as_longlong(s) & 0x7FF0000000000000ull;
       const double lo = __longlong_as_double((long long)e);
       const double lo1 = s > 0.0 ? __longlong_as_double((long long)(e | 1)) : 0.0;
@@ -286,8 +291,9 @@ __device__ inline double cx_rms_seq_sum_wg(const float* x, uint32_t n) {
           if (g < quads) {
 #pragma unroll
             for (uint32_t j = 0; j < 4; j++) {
-              a0 += t[4 * g + j];
-              a1 += t[4 * g + j];
+              const double v = t[4 * g + j];
+              a0 += v * v;
+              a1 += v * v;
             }
           }
         r.d0 = a0 - lo;
@@ -318,7 +324,8 @@ __device__ inline double cx_rms_seq_sum_wg(const float* x, uint32_t n) {
         if (out) {
           double a = before;
 #pragma unroll
-          for (uint32_t j = 0; j < 16; j++) a += t[j];  // (values past the run are +0.0)
+          for (uint32_t j = 0; j < 16; j++)  // (values past the run are 0)
+            a += (double)t[j] * (double)t[j];
           wsum[w] = a;
         } else {
           wsum[w] = after;
@@ -337,11 +344,21 @@ __device__ inline double cx_rms_seq_sum_wg(const float* x, uint32_t n) {
   return s;
 }
 
+// Which of the two sums in order a launch over rows of n values takes (the
+// template parameter WG below): the workgroup's from where its rounds, one a
+// binade, cost less than the wave's adds. Wave and workgroup, us, rows that all
+// need the sum: one row of 896 values 8.8, 7.9, of 1024 9.6, 10.2, of 1152 10.7,
+// 9.4; 512 rows of 896 9.9, 9.6, of 1024 10.7, 12.3, of 1152 11.6, 11.6, of 2048
+// 18.5, 14.2; 1000 rows of 896 10.7, 12.4. N(0, 1) rows, 8000 of 1152 24.1, 24.2,
+// of 2048 38.3, 34.4.
+inline bool cx_rms_wg(size_t n) { return n > 1024; }
+
 // The rmsnorm factor of x[0..n) (n % 4 == 0, x 16-byte aligned) over a
 // 256-thread workgroup, bit for bit the reference's: the tree (4 values a
 // lane, wave sums, ((w0 + w1) + w2) + w3), the check above, and the sum in
-// order when the check asks for it. `red` is 8 doubles and `flag` an int of
+// order when the check asks for it. `red` is 9 doubles and `flag` an int of
 // shared memory; every thread of the workgroup calls it.
+template <bool WG>
 __device__ inline double cx_rms_scale(const float* x, uint32_t n, float eps, double* red,
                                       int* flag) {
   const int tid = threadIdx.x;
@@ -374,7 +391,16 @@ __device__ inline double cx_rms_scale(const float* x, uint32_t n, float eps, dou
   if (reach && risk.unsure(reach)) *flag = 1;
   __syncthreads();
   if (*flag) {  // the same for every thread
-    scale = cx_rms_factor(cx_rms_seq_sum_wg(x, n), n, eps);
+    if constexpr (WG) {
+      scale = cx_rms_factor(cx_rms_seq_sum_wg(x, n), n, eps);
+    } else {
+      if (tid < 64) {
+        const double seq = cx_rms_seq_sum(x, n);
+        if (tid == 0) red[8] = seq;
+      }
+      __syncthreads();
+      scale = cx_rms_factor(red[8], n, eps);
+    }
   }
   __syncthreads();  // red and flag are free again
   return scale;

@@ -1094,17 +1094,17 @@ __global__ __launch_bounds__(256) void k_quantize_gemm(const float* x, uint32_t 
 // one workgroup a row; and silu(g) * u (src/forward.rs:483-487); each
 // value is what the row kernel writes, then quantized as k_quantize_gemm
 // quantizes it. Rows [m, m_pad) are zero.
-template <int SUB>
+template <int SUB, bool WG>
 __global__ __launch_bounds__(256) void k_norm_quant_gemm(const float* x, const float* w,
                                                          uint32_t m, uint32_t k, float eps,
                                                          uint32_t m_pad, int8_t* xq, float* xexs) {
-  __shared__ double red[8];
+  __shared__ double red[9];
   __shared__ int flag;
   const int tid = threadIdx.x;
   const uint32_t a = blockIdx.x;
   const float* xr = x + (size_t)a * k;
   double scale = 0.0;
-  if (a < m) scale = cx_rms_scale(xr, k, eps, red, &flag);  // the same for the whole workgroup
+  if (a < m) scale = cx_rms_scale<WG>(xr, k, eps, red, &flag);  // the same for the whole workgroup
   for (uint32_t i = 8 * tid; i < k; i += 2048) {  // whole quads of lanes (k % 32 == 0)
     float v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (a < m) {
@@ -1369,12 +1369,11 @@ int cx_gemm_norm_quantize(const float* x, const float* w, size_t m, size_t k, fl
   if (!m) return CX_OK;
   const uint32_t mp = pad64(m);
   uint8_t* sc = reinterpret_cast<uint8_t*>(scratch);
-  if (sub == 16)
-    hipLaunchKernelGGL(k_norm_quant_gemm<16>, dim3(mp), dim3(256), 0, s, x, w, (uint32_t)m,
-                       (uint32_t)k, eps, mp, scratch_xq(sc), scratch_xexs(sc, mp, k));
-  else
-    hipLaunchKernelGGL(k_norm_quant_gemm<32>, dim3(mp), dim3(256), 0, s, x, w, (uint32_t)m,
-                       (uint32_t)k, eps, mp, scratch_xq(sc), scratch_xexs(sc, mp, k));
+  const bool wg = cx_rms_wg(k);
+  const auto norm = sub == 16 ? (wg ? k_norm_quant_gemm<16, true> : k_norm_quant_gemm<16, false>)
+                              : (wg ? k_norm_quant_gemm<32, true> : k_norm_quant_gemm<32, false>);
+  hipLaunchKernelGGL(norm, dim3(mp), dim3(256), 0, s, x, w, (uint32_t)m, (uint32_t)k, eps, mp,
+                     scratch_xq(sc), scratch_xexs(sc, mp, k));
   CX_HIP(hipGetLastError());
   return CX_OK;
 }

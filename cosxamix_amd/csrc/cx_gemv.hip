@@ -2474,12 +2474,12 @@ __global__ __launch_bounds__(256) void k_swiglu_quant(const float* g, const floa
 
 // rmsnorm (src/kernels/scalar.rs:40-53) of one row, then its quantization:
 // (x as f64 * scale) as f32 * w
-template <int SUB>
+template <int SUB, bool WG>
 __global__ __launch_bounds__(256) void k_norm_quant(const float* x, const float* w, uint32_t n,
                                                     float eps, int8_t* xq, float* xe, float* xs) {
-  __shared__ double red[8];
+  __shared__ double red[9];
   __shared__ int flag;
-  const double scale = cx_rms_scale(x, n, eps, red, &flag);
+  const double scale = cx_rms_scale<WG>(x, n, eps, red, &flag);
   for (uint32_t i = 8 * threadIdx.x; i < n; i += 8 * 256) {  // n % SUB == 0: whole groups
     float v[8], nw[8];
     cx_load8(x + i, v);
@@ -2494,14 +2494,15 @@ __global__ __launch_bounds__(256) void k_norm_quant(const float* x, const float*
 // (cx_rms_scale, bit for bit), then v = (x as f64 * scale) as f32 * w, the
 // values the decode step's fused GEMV quantizes for the same row, so a
 // batched prefill matches token-by-token decoding.
+template <bool WG>
 __global__ __launch_bounds__(256) void k_norm_rows(const float* x, const float* w, uint32_t k,
                                                    float eps, float* out) {
-  __shared__ double red[8];
+  __shared__ double red[9];
   __shared__ int flag;
   const int tid = threadIdx.x;
   const float* xr = x + (size_t)blockIdx.x * k;
   float* yr = out + (size_t)blockIdx.x * k;
-  const double scale = cx_rms_scale(xr, k, eps, red, &flag);
+  const double scale = cx_rms_scale<WG>(xr, k, eps, red, &flag);
   for (uint32_t i = 8 * tid; i < k; i += 2048) {
     float v[8], nw[8];
     cx_load8(xr + i, v);
@@ -2538,13 +2539,14 @@ __global__ __launch_bounds__(256) void k_add_rows(float* y, const float* a, uint
   y[i] = y[i] + a[(r % a_rows) * n + i % n];
 }
 
+template <bool WG>
 __global__ __launch_bounds__(256) void k_rmsnorm(float* out, const float* in, const float* w,
                                                  uint32_t n, float eps) {
-  __shared__ double red[8];
+  __shared__ double red[9];
   __shared__ int flag;
   const float* x = in + (size_t)blockIdx.x * n;
   float* y = out + (size_t)blockIdx.x * n;
-  const double scale = cx_rms_scale(x, n, eps, red, &flag);
+  const double scale = cx_rms_scale<WG>(x, n, eps, red, &flag);
   for (uint32_t i = threadIdx.x; i < n; i += 256) y[i] = (float)((double)x[i] * scale) * w[i];
 }
 }  // namespace
@@ -2586,10 +2588,10 @@ int cx_launch_norm_quant(const float* x, const float* w, size_t n, float eps, in
   CX_REQUIRE(sub == 16 || sub == 32, "norm: sub must be 16 or 32, got %d", sub);
   CX_REQUIRE(n % (size_t)sub == 0 && n < (1u << 31), "norm: width %zu must be whole sub-blocks of %d",
              n, sub);
-  if (sub == 16)
-    hipLaunchKernelGGL(k_norm_quant<16>, dim3(1), dim3(256), 0, s, x, w, (uint32_t)n, eps, xq, xe, xs);
-  else
-    hipLaunchKernelGGL(k_norm_quant<32>, dim3(1), dim3(256), 0, s, x, w, (uint32_t)n, eps, xq, xe, xs);
+  const bool wg = cx_rms_wg(n);
+  const auto norm = sub == 16 ? (wg ? k_norm_quant<16, true> : k_norm_quant<16, false>)
+                              : (wg ? k_norm_quant<32, true> : k_norm_quant<32, false>);
+  hipLaunchKernelGGL(norm, dim3(1), dim3(256), 0, s, x, w, (uint32_t)n, eps, xq, xe, xs);
   CX_HIP(hipGetLastError());
   return CX_OK;
 }
@@ -2599,8 +2601,8 @@ int cx_launch_norm_rows(const float* x, const float* w, size_t rows, size_t k, f
   CX_REQUIRE(x && w && out, "norm rows: null pointer");
   CX_REQUIRE(k % 8 == 0 && rows < (1u << 31), "norm rows: %zu x %zu", rows, k);
   if (!rows || !k) return CX_OK;
-  hipLaunchKernelGGL(k_norm_rows, dim3((unsigned)rows), dim3(256), 0, s, x, w, (uint32_t)k, eps,
-                     out);
+  hipLaunchKernelGGL(cx_rms_wg(k) ? k_norm_rows<true> : k_norm_rows<false>, dim3((unsigned)rows),
+                     dim3(256), 0, s, x, w, (uint32_t)k, eps, out);
   CX_HIP(hipGetLastError());
   return CX_OK;
 }
@@ -2633,7 +2635,8 @@ int cx_launch_rmsnorm(float* out, const float* in, const float* w, size_t rows, 
   CX_REQUIRE(out && in && w, "rmsnorm: null pointer");
   CX_REQUIRE(n % 4 == 0, "rmsnorm: n=%zu must be a multiple of 4", n);
   if (!rows || !n) return CX_OK;
-  hipLaunchKernelGGL(k_rmsnorm, dim3((unsigned)rows), dim3(256), 0, s, out, in, w, (uint32_t)n, eps);
+  hipLaunchKernelGGL(cx_rms_wg(n) ? k_rmsnorm<true> : k_rmsnorm<false>, dim3((unsigned)rows),
+                     dim3(256), 0, s, out, in, w, (uint32_t)n, eps);
   CX_HIP(hipGetLastError());
   return CX_OK;
 }

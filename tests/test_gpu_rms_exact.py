@@ -45,6 +45,31 @@ def test_rmsnorm_operator_on_splitting_vectors(dev, n):
         assert np.array_equal(got[r].view(np.uint32), want.view(np.uint32)), r
 
 
+@pytest.mark.parametrize("n", [896, 1024, 1028, 1152, 2048, 4096, 4228, 11008])
+def test_rmsnorm_operator_where_the_sum_is_hard_to_follow(dev, n):
+    """Rows that all take the sum in order (one output is an f32 subnormal, which
+    the check never lets pass): a sum still 0 after hundreds of values, one that
+    changes its binade all along, halfway cases of its last bit. 1024 is the
+    longest row of the wave's sum, 1028 the shortest of the workgroup's."""
+    from cosxamix_amd import ops
+    from test_rms_order_model import _vectors
+    rows = []
+    for x in _vectors(n):
+        x = x.astype(np.float32)
+        x[n // 2] = np.float32(1e-42) * (1 + np.abs(x).max())  # 0 < its output < 2^-126
+        rows.append(x)
+    x = np.stack(rows)
+    w = np.random.default_rng(n).normal(1.0, 0.1, n).astype(np.float32)
+    out = torch.empty(x.size, device=dev)
+    ops.rmsnorm(out, torch.from_numpy(x.ravel()).to(dev), torch.from_numpy(w).to(dev), 1e-6)
+    got = out.cpu().numpy().reshape(x.shape)
+    for r in range(len(x)):
+        want = O.rmsnorm(x[r], w, 1e-6)
+        v = float(x[r, n // 2]) * R.factor(R.seq_sum(x[r]), n, 1e-6)
+        assert 0 < v < 2.0 ** -126, r
+        assert np.array_equal(got[r].view(np.uint32), want.view(np.uint32)), r
+
+
 CASES = [
     ("2048-q4k", dict(capas=1, dim=2048, cabezas=16, cabezas_kv=2, ffn=1024, vocab=300,
                       contexto=64), O.Q4_K, O.Q4_K),
