@@ -681,7 +681,10 @@ __device__ inline uint2 less(uint2 v, uint32_t off) {
 }
 
 // Members: load(), this lane's words of the stage at p, of which `left` blocks are
-// in the row (a block past them reads the last); pin(); scales(), the factors of
+// in the row (words of a block past them are left as they are, no term uses them: a
+// row of 32 to 400 values waited for eight blocks' loads, and for the last stage's
+// twice. Q5_0 4864 x 96, m = 64, 14.3 -> 11.0 us, x 288 19.3 -> 14.5; Q8_0 4864 x
+// 896, m = 512, 31.0 -> 29.5); pin(); scales(), the factors of
 // this lane's sub-blocks PL G .. + PL (MIN: and their minima); operand(), its bytes
 // 8 G .. + 8 of the stage's 32-value group gg.
 template <int T> struct XQ;
@@ -795,7 +798,7 @@ template <> struct XQ<CX_Q8_0> {
   __device__ void load(const uint8_t* p, int G, uint32_t left) {
 #pragma unroll
     for (uint32_t i = 0; i < 8; i++)
-      q[i] = at2x2(p + (i < left ? i : left - 1) * BPB + 2 + 8 * G);
+      if (i < left) q[i] = at2x2(p + i * BPB + 2 + 8 * G);
 #pragma unroll
     for (uint32_t i = 0; i < 2; i++)
       d[i] = *reinterpret_cast<const uint16_t*>(p + min(2 * G + i, left - 1) * BPB);
@@ -825,9 +828,11 @@ template <> struct XQ<CX_Q5_0> {
   __device__ void load(const uint8_t* p, int G, uint32_t left) {
 #pragma unroll
     for (uint32_t i = 0; i < 8; i++) {
-      const uint8_t* b = p + (i < left ? i : left - 1) * BPB;
-      q[i] = at2x2(b + 6 + 8 * (G & 1));
-      h[i] = b[2 + G];
+      if (i < left) {
+        const uint8_t* b = p + i * BPB;
+        q[i] = at2x2(b + 6 + 8 * (G & 1));
+        h[i] = b[2 + G];
+      }
     }
 #pragma unroll
     for (uint32_t i = 0; i < 2; i++)
@@ -932,7 +937,7 @@ __global__ __launch_bounds__(256, OCC) void k_gemm_x(GemmParams P) {
   for (int t = 0; t < WA; t++)
 #pragma unroll
     for (int i = 0; i < 4; i++) acc[t][i] = 0.0f;
-  Q wn;
+  Q wn{};  // (words that a short row never loads)
   wn.load(wrow, G, P.nb);
   issue(0);
   const uint32_t half = G < 2 ? ~0u : 0u;  // (16-value sub-blocks)
@@ -943,9 +948,10 @@ __global__ __launch_bounds__(256, OCC) void k_gemm_x(GemmParams P) {
     cx_barrier();     // every wave's part; stage sb - 1 is read
     Q w = wn;
     w.arrived();  // before the next loads are issued, as in k_gemm_w
-    if (sb + 1 < nst) issue(sb + 1);
-    const uint32_t sn = sb + 1 < nst ? sb + 1 : sb;
-    wn.load(wrow + (size_t)sn * (Q::NB * Q::BPB), G, P.nb - sn * Q::NB);
+    if (sb + 1 < nst) {
+      issue(sb + 1);
+      wn.load(wrow + (size_t)(sb + 1) * (Q::NB * Q::BPB), G, P.nb - (sb + 1) * Q::NB);
+    }
     const uint8_t* X = lds + (sb & 1) * SH::STAGE;
     const float* E = reinterpret_cast<const float*>(X + 256 * MT) + 4 * G;
     const uint32_t ng = Q::NB == 1 ? 8 : P.nb - sb * Q::NB;  // 32-value groups (more than 8: 8)
