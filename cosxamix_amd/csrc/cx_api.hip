@@ -1562,16 +1562,17 @@ static int run_steps(cx_cache* C, size_t prompt_end, size_t steps, float* step_m
 // ------------------------------------------------------ batched prefill
 // Modelo::forward over several tokens (src/forward.rs:375-505) as one pass
 // per layer over a chunk of up to T tokens. The GEMVs become the int8 MFMA
-// contraction for Q4_K/Q5_K (other types run the GEMV row by row), and the
-// attention takes the chunk's tokens at once. Every value equals what token-by-token decoding computes:
+// contraction, and the attention takes the chunk's tokens at once. Every value
+// equals what token-by-token decoding computes:
 // - the contraction is bit-identical to the GEMV;
 // - the rows are normalized in the fused GEMV prologue's tree;
 // - the quantization of a row is a function of its values alone;
 // - bias and residual adds are the same single f32 adds as the epilogues;
 // - the attention forms every score, softmax and output in the one-token
-//   kernels' order (cx_attn_many.hip for a full chunk, else the decode step's
-//   kernels with several query tokens).
+//   kernels' order (cx_attn_many.hip where the chunk is long enough for it, else
+//   the decode step's kernels with several query tokens).
 // So a prompt gives the same logits, cache and tokens either way.
+
 // Tokens a chunk. 512 rather than 256: the attention of many tokens spreads its
 // outputs (tokens x heads x head_dim) over the chip, and the contraction's tiles
 // fill more CUs.
@@ -1645,29 +1646,19 @@ static int prefill_alloc(cx_cache* C) {
   return rc ? prefill_alloc_chunk(C, kPrefillShortT, kPrefillShortBytes) : rc;
 }
 
-// out[r] = W . in[r] for `rows` rows of width k: the MFMA contraction,
-// quantizing `in` unless *quantized (the sub-block size an earlier call of
-// the same input quantized with, or 0) already matches the type's; the GEMV
-// row by row on the step's activation buffers otherwise.
+// out[r] = W . in[r] for `rows` rows of width k by the MFMA contraction (every
+// type a model's matrices have), quantizing `in` unless *quantized (the sub-block
+// size an earlier call of the same input quantized with, or 0) already matches
+// the type's.
 static int prefill_matmul(cx_cache* C, int type, const uint8_t* w, uint32_t n, uint32_t k,
                           const float* in, uint32_t rows, float* out, int* quantized) {
-  cx_model* m = C->m;
-  hipStream_t s = m->stream;
+  CX_REQUIRE(cx_gemm_supported(type), "prefill: type %d has no quantized path here", type);
+  const int sub = cx_sub(type);
+  hipStream_t s = C->m->stream;
   int rc;
-  if (cx_gemm_supported(type)) {
-    const int sub = cx_sub(type);
-    if (*quantized != sub && (rc = cx_gemm_quantize(in, rows, k, sub, C->pf.scratch, s))) return rc;
-    *quantized = sub;
-    return cx_gemm_apply(type, w, n, k, rows, out, C->pf.scratch, s);
-  }
-  const cx_qact act{m->xq, m->xe, m->xs};
-  for (uint32_t r = 0; r < rows; r++) {
-    if ((rc = cx_launch_quantize(in + (size_t)r * k, 1, k, cx_sub(type), m->xq, m->xe, m->xs, s)))
-      return rc;
-    cx_seg seg{w, out + (size_t)r * n, nullptr, n};
-    if ((rc = cx_launch_gemv(type, &seg, 1, k, act, CX_EPI_STORE, nullptr, s))) return rc;
-  }
-  return CX_OK;
+  if (*quantized != sub && (rc = cx_gemm_quantize(in, rows, k, sub, C->pf.scratch, s))) return rc;
+  *quantized = sub;
+  return cx_gemm_apply(type, w, n, k, rows, out, C->pf.scratch, s);
 }
 
 // out[i] = in . w[i]^T (+ bias[i]) for `count` matrices over one input
