@@ -97,14 +97,14 @@ def test_forward_logits_and_greedy_tokens_match_oracle(F, name, cfg, t, tdown):
 VARIED = [
     # (name, config, linear type, down type, prompt length); k = 2048: the
     # row kernels' fused rmsnorm (q/k/v, gate/up/SwiGLU); k = 4096: the LDS
-    # gate/up/SwiGLU kernel; a 300-token prompt: two prefill chunks of the
+    # gate/up/SwiGLU kernel; a 530-token prompt: two prefill chunks of the
     # MFMA contraction's fused rmsnorm; 896: the 32-value block kernels
     ("2048-q4k", dict(capas=2, dim=2048, cabezas=16, cabezas_kv=2, ffn=11008, vocab=3000,
                       contexto=200, rope=1e6), O.Q4_K, O.Q4_K, 24),
     ("4096-q4k-q5kdown", dict(capas=2, dim=4096, cabezas=32, cabezas_kv=8, ffn=14336,
                               vocab=2000, contexto=200, rope=5e5), O.Q4_K, O.Q5_K, 24),
-    ("2048-q5k-q3kdown-300", dict(capas=2, dim=2048, cabezas=16, cabezas_kv=2, ffn=1024,
-                                  vocab=1000, contexto=400, rope=1e6), O.Q5_K, O.Q3_K, 300),
+    ("2048-q5k-q3kdown-530", dict(capas=2, dim=2048, cabezas=16, cabezas_kv=2, ffn=1024,
+                                  vocab=1000, contexto=600, rope=1e6), O.Q5_K, O.Q3_K, 530),
     ("512-q2k-q3kdown", dict(capas=2, dim=512, cabezas=8, cabezas_kv=2, ffn=1536, vocab=1500,
                              contexto=200, rope=10000.0), O.Q2_K, O.Q3_K, 24),
     ("896-q8_0", dict(capas=2, dim=896, cabezas=14, cabezas_kv=2, ffn=4864, vocab=640,
