@@ -1,9 +1,10 @@
 """Attention of many query tokens (cx_attn_many.hip) through ops.atencion, bit
 for bit against the oracle's ops::atencion (src/ops.rs:1258-1325), at the edges of
 its tiles: rows (tokens x heads per group) around 64 and 128, positions around 32,
-64 and 128, one to sixteen heads per group, both head dims, and every row count a
-lane takes. Values that a row does not see may be anything; a captured call and
-misaligned rows take the general kernel."""
+64 and 128, one to sixteen heads per group, both head dims, every score tile and
+every row count a lane takes, and calls of several slabs. Values that a row does
+not see may be anything; a captured call and misaligned tensors take the general
+kernel; the scores' buffer is no captured graph's."""
 import ctypes as C
 
 import numpy as np
@@ -50,13 +51,28 @@ def test_many_tokens_bit_exact(dev, tokens, total, heads, kv, hd):
     assert same(run(dev, q, k, v, heads, kv, hd), oracle(q, k, v, heads, kv, hd))
 
 
-def test_large_tiles_bit_exact(dev):
-    # 128 x 128 score tiles and four rows a lane: the first and last tokens
-    # against the oracle (each is the last token of its own prefix)
-    tokens, total, heads, kv, hd = 512, 1030, 32, 8, 128
+def tile_and_rows(tokens, total, heads, kv, hd):
+    """The launch's choice (cx_attn_many.hip): score tile, P.V rows a lane"""
+    rows = tokens * (heads // kv)
+    tile = 128 if -(-rows // 128) * -(-total // 128) * kv >= 1024 else 64
+    one = -(-rows // (1024 // hd)) * kv  # workgroups of one row a lane
+    return tile, 4 if one // 4 >= 512 else 2 if one // 2 >= 256 else 1
+
+
+# every score tile and P.V row count of both head dims that the sizes above (64 x
+# 64 tiles, one row a lane at head_dim 64) leave out: the first and last tokens
+# against the oracle (each is the last token of its own prefix), and those beside
+# the edges of tiles
+@pytest.mark.parametrize("tokens,total,heads,kv,hd,tile,rows", [
+    (512, 1030, 32, 8, 128, 128, 4), (512, 600, 32, 8, 128, 64, 4), (300, 1100, 16, 2, 128, 64, 2),
+    (300, 4200, 16, 2, 128, 128, 2), (130, 8300, 8, 8, 128, 128, 1),
+    (1200, 1200, 14, 2, 64, 128, 2), (2600, 2600, 14, 2, 64, 128, 4),
+    (700, 1100, 14, 2, 64, 64, 2), (512, 5000, 14, 2, 64, 128, 1)])
+def test_large_tiles_bit_exact(dev, tokens, total, heads, kv, hd, tile, rows):
+    assert tile_and_rows(tokens, total, heads, kv, hd) == (tile, rows)
     q, k, v = inputs(5, tokens, total, heads, kv, hd)
     got = run(dev, q, k, v, heads, kv, hd)
-    for t in (0, 1, 31, 32, 300, 510, 511):
+    for t in (0, 1, 31, 32, tokens // 2 + 7, tokens - 2, tokens - 1):
         n = total - tokens + t + 1
         assert same(got[t], oracle(q[t:t + 1], k[:n], v[:n], heads, kv, hd)), t
 
