@@ -204,7 +204,7 @@ __device__ inline double cx_rms_seq_sum(const float* x, uint32_t n) {
 // The same sum by a 256-thread workgroup (n % 4 == 0, x 16-byte aligned, every
 // x finite), without one dependent add a value. A launch over
 // 512 rows lasts as long as its rows that take this sum: k_norm_quant_gemm
-// at k = 2048 17.7 -> 12.3 us, at 4096 35.9 -> 17.1 (5.3 where no row does).
+// at k = 2048 17.7 -> 11.8 us, at 4096 35.9 -> 16.9 (5.3 where no row does).
 // What bounds it is the chain of its rounds, one for each binade.
 //
 // While the running sum s stays in one binade [2^E, 2^(E+1)), whose f64 values

@@ -478,7 +478,9 @@ int launch(const cx_attn_many_args& a, hipStream_t s) {
 // T = 128 770, 745, T = 256 1081, 1124; after 7000 T = 64 2177, 1878, T = 128
 // 2462, 3290; 8B shape after 60 T = 64 1287, 1249, T = 128 2125, 2145, after 7000
 // T = 32 2527, 3201; 0.5B shape after 60 T = 256 1233, 1233, after 7000 T = 128
-// 2558, 2232, T = 256 2880, 3664.
+// 2558, 2232, T = 256 2880, 3664. The product of tokens and width does not decide
+// alone: the line gives up the 8B shape's T = 32 after 7000 positions, whose product
+// is that of the 3B shape's T = 64, which the other kernels serve better.
 bool cx_attn_many_suits_prefill(size_t tokens, size_t total, size_t heads, size_t hd) {
   return (hd == 64 || hd == 128) &&
          tokens * heads * hd >= (total < 1024 ? 320 * 1024 : 176 * 1024);

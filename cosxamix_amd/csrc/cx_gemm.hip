@@ -16,8 +16,8 @@
 // order makes a batched prefill bit-identical to token-by-token.
 //
 // The per-sub-block f32 term (6 VALU operations per output and sub-block in
-// k_gemm, 5 in k_gemm_w) bounds this path, not the MFMA: a 16x16x32 MFMA is
-// followed by 24 or 20 VALU instructions per lane.
+// k_gemm, 5 in k_gemm_w) is most of this path's work, not the MFMA: a 16x16x32
+// MFMA is followed by 24 or 20 VALU instructions per lane.
 //
 // MFMA lane layout (checked on the device): A 16x32 — lane l holds row
 // l%16, k = 8(l/16)..+8 as 8 bytes; B 32x16 — lane l holds column l%16,
@@ -398,10 +398,12 @@ __global__ __launch_bounds__(64 * RW * AW * KS) void k_gemm(GemmParams P) {
 // zero may come out with the other sign; it is added to a sum that starts at
 // +0.0, which no zero changes.)
 //
-// The VALU bounds it: 5 operations an output and sub-block at ~2.5 clocks, of which
-// the four at a time that one wave can have ready run at ~3.1 with three waves a
-// SIMD. 11008 x 2048, m = 512: 84 -> 79 us (k_gemm 64 x 64), 32.8 waves' worth of
-// terms at that rate are 60; the rest is the last round of workgroups (1.8 a CU).
+// What bounds it, by counters (11008 x 2048, m = 512, 74 us at 2.24 GHz): 35.4 M
+// VALU instructions, 34.6 k a SIMD, of which the terms are 27.5 k. At the 2.5 to 3.1
+// clocks an instruction that two to three waves a SIMD reach they are 39 to 48 us. Of
+// the waves' time 32% waits to issue and 24% for loads, LDS and the barrier of every
+// super-block, and the 1376 workgroups are 1.8 rounds of 768. 2048 x 11008: 39.0 M
+// instructions in 88 us, 512 workgroups, two waves a SIMD.
 // Measured beside it and dropped: weights as the A operand with the scales in an
 // LDS table (no better), 12 and 16 waves a workgroup (slower: the barrier), scales
 // by DPP or in SGPRs (conversions and scalar loads cost what they save).
@@ -661,6 +663,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_gemm_w(GemmParams P) {
 // per-row kernel's (float)E - 32.0f * xs is, and the term is (xe * scale) * E' as
 // there. The MFMA starts from the bits of E_BASE, so that E' as f32 is one
 // subtraction at full rate, not a conversion at half (|E'| < 2^22: exact).
+//
+// With few rows the round trip of a stage bounds it: Q6_K 2048 x 11008, m = 77, is
+// 160 workgroups, one wave a SIMD, and 43 stages of 1.8 us (77.7 us), 9 clocks an
+// instruction; by m = 8 nothing is shorter.
 typedef uint32_t u32_at2 __attribute__((aligned(2)));  // a word at any even address
 __device__ inline uint32_t at2(const uint8_t* p) { return *reinterpret_cast<const u32_at2*>(p); }
 __device__ inline uint2 at2x2(const uint8_t* p) {
@@ -1183,8 +1189,7 @@ Config make_config_w(gemm_kernel* k) {
 }
 
 // The tile shapes: weight rows x activation rows, waves, super-blocks per
-// stage, ring stages. 0 to 5 (k_gemm) are each the fastest of a sweep for some
-// (n, m) of 11008 x 2048 and 2048 x 11008, m = 2 .. 512; 6 to 8 are k_gemm_w.
+// stage, ring stages: 0 to 5 are k_gemm, 6 to 8 k_gemm_w.
 template <int T>
 Config config(int id, gemm_kernel* k) {
   switch (id) {
@@ -1201,22 +1206,25 @@ Config config(int id, gemm_kernel* k) {
 }
 
 // Weights in registers (k_gemm_w) where its tiles give the chip enough
-// workgroups, the larger tile first; measured against the best k_gemm tile, us:
-//   64 x 64: 11008 x 2048 m = 512 79, 83, m = 256 48, 57; 14336 x 4096 m = 512 161,
-//     181, m = 128 57, 64; 4096 x 4096 m = 512 62, 69
-//   64 x 32: 11008 x 2048 m = 128 34, 39; 4096 x 4096 m = 256 42, 63; 2048 x 11008
-//     m = 512 93, 100 (its 512 workgroups; at m = 256 79, 69: k_gemm)
-//   64 x 16: 4096 x 4096 m = 64 28, 40, m = 128 32, 62; 4096 x 14336 (Q5_K) m = 32
-//     78, 85; 2048 x 11008 m = 128 58, 55, 1847 x 2048 m = 389 38, 28: k_gemm
-// Otherwise, with m <= 16 rows of many weights, 64 x 16 of k_gemm (11008 x 2048 18.4
-// against 18.9), and for few weight rows (n < 4096: 2048 x 11008 and the q/o/k/v
+// workgroups, the larger tile first. Whole calls (the quantization with it), us,
+// Q4_K, beside the best of k_gemm's tiles:
+//   64 x 64: 11008 x 2048 m = 512 73, 103, m = 256 45, 59; 4096 x 4096 m = 512 58, 75
+//   64 x 32: 11008 x 2048 m = 128 31, 36; 4096 x 4096 m = 256 39, 42; 2048 x 11008
+//     m = 512 88, 96 (its 512 workgroups; at m = 256 76, 66: k_gemm)
+//   64 x 16: no better than k_gemm's 64 x 16 and 64 x 32, and no worse than by 10%:
+//     4096 x 4096 m = 64 26.5, 26.3, m = 128 29.9, 30.2; 4096 x 14336 (Q5_K) m = 64
+//     78, 71; 2048 x 11008 m = 128 57, 54, 1847 x 2048 m = 389 33, 26: k_gemm
+// Otherwise, with m <= 16 rows of many weights, 64 x 16 of k_gemm (11008 x 2048 17.9;
+// 16 x 16 20.8), and for few weight rows (n < 4096: 2048 x 11008 and the q/o/k/v
 // shapes) the largest k_gemm tile (64 x 64, 64 x 32, then 32 x 32) that gives at
 // least 5/8 of the CUs a workgroup; below that, 16 x 16 tiles that split k over the
-// waves (four super-blocks a stage up to a workgroup per CU, two past it). Swept at
-// n = 2048 (k = 2048 and 11008) and n = 256 for m = 64 to 512: the rule picks the
-// fastest tile or one within 3% of it; at m = 256 2048 x 11008 takes 62 us in 64 x 32
-// tiles against 88 in 64 x 64, 2048 x 2048 16.3 against 20.6, 256 x 2048 9.5 in 16 x
-// 16 against 20.8.
+// waves (four super-blocks a stage up to a workgroup per CU, two past it): 2048 x
+// 11008 m = 256 66 us in 64 x 32 tiles, 90 in 64 x 64, 2048 x 2048 20.4, 24.7, 256 x
+// 2048 13.4 in 16 x 16, 24.8. Within 5% of the best tile there but for m = 389 of
+// 2048 x 11008 (94; 64 x 32 of k_gemm_w 85).
+// Where n >= 4096 and k is long the line at 16 rows costs: 4096 x 4096, m <= 16, 26
+// us where 16 x 16 tiles over a split k take 15.6, 4096 x 14336 65 and 29 (m = 17 to
+// 32 69 and 48).
 int choose(uint32_t n, uint32_t m) {
   auto tiles = [&](uint32_t tw, uint32_t mt) { return (n + tw - 1) / tw * ((m + mt - 1) / mt); };
   const bool few = n < 4096;
@@ -1267,13 +1275,19 @@ Config make_config_x(gemm_kernel* k) {
   return Config{SH::TW, SH::MT, 256, SH::lds};
 }
 
-// The largest tile whose workgroups still keep the chip busy; us with 16, 32, 64
-// activation rows a workgroup (Q6_K, then Q8_0 whose term is shorter):
-//   Q6_K 4096 x 14336 m = 512 460, 303, 276, m = 256 249, 179, 209; 11008 x 2048
-//   m = 128 59, 45, 48, m = 17 28, 29, 38; 2048 x 11008 m = 256 137, 118, 165,
-//   m = 128 87, 112, 162
-//   Q8_0 4864 x 896 m = 512 56, 38, 32, m = 128 24, 22, 22; 2048 x 2048 m = 512 67,
-//   43, 33, m = 256 40, 29, 32, m = 128 27, 27, 31; 896 x 4864 m = 512 62, 50, 61
+// The largest tile whose workgroups still keep the chip busy; whole calls, us, with
+// 16, 32, 64 activation rows a workgroup (the 32-value formats' term is shorter):
+//   Q6_K 4096 x 14336 m = 512 437, 285, 253, m = 256 237, 169, 203; 11008 x 2048
+//   m = 128 52, 41, 45, m = 17 26, 26, 36; 2048 x 11008 m = 256 128, 112, 164,
+//   m = 128 88, 111, 163
+//   Q8_0 4864 x 896 m = 512 44, 31, 29, m = 128 21.5, 19.5, 19.7; 2048 x 2048
+//   m = 512 61, 39, 32, m = 256 37, 27, 31; 896 x 4864 m = 512 60, 48, 60
+//   Q5_0 4864 x 896 m = 512 64, 41, 35, m = 128 28, 24, 23; 2048 x 2048 m = 512 89,
+//   53, 39
+// Q6_K, Q8_0 and Q5_0 are within 5% of their best tile over these widths and m = 17
+// to 512. Q2_K and Q3_K keep 16 rows longer, which this rule does not know:
+//   Q2_K 4096 x 14336 m = 77 105, 139, 236, 2048 x 11008 m = 256 90, 113, 185 (both
+//   take 32: 1.36 and 1.28 of the best); Q3_K 95, 120, 188 and 89, 102, 150
 template <int T>
 Config config_x(uint32_t n, uint32_t m, gemm_kernel* k) {
   auto tiles = [&](uint32_t mt) { return (n + 63) / 64 * ((m + mt - 1) / mt); };
