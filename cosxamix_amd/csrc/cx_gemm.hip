@@ -665,7 +665,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_gemm_w(GemmParams P) {
 // subtraction at full rate, not a conversion at half (|E'| < 2^22: exact).
 //
 // With few rows the round trip of a stage bounds it: Q6_K 2048 x 11008, m = 77, is
-// 160 workgroups, one wave a SIMD, and 43 stages of 1.8 us (77.7 us), 9 clocks an
+// 160 workgroups, one wave a SIMD, and 43 stages of 1.8 us (77.7 us), 11 clocks an
 // instruction; by m = 8 nothing is shorter.
 typedef uint32_t u32_at2 __attribute__((aligned(2)));  // a word at any even address
 __device__ inline uint32_t at2(const uint8_t* p) { return *reinterpret_cast<const u32_at2*>(p); }
@@ -1222,9 +1222,10 @@ Config config(int id, gemm_kernel* k) {
 // 11008 m = 256 66 us in 64 x 32 tiles, 90 in 64 x 64, 2048 x 2048 20.4, 24.7, 256 x
 // 2048 13.4 in 16 x 16, 24.8. Within 5% of the best tile there but for m = 389 of
 // 2048 x 11008 (94; 64 x 32 of k_gemm_w 85).
-// Where n >= 4096 and k is long the line at 16 rows costs: 4096 x 4096, m <= 16, 26
-// us where 16 x 16 tiles over a split k take 15.6, 4096 x 14336 65 and 29 (m = 17 to
-// 32 69 and 48).
+// Where n >= 4096 the line at 16 rows costs, most where k is long: 4096 x 4096, m <=
+// 16, 26 us where 16 x 16 tiles over a split k take 15.6, 4096 x 14336 65 and 29 (m =
+// 17 to 32 69 and 48), 8192 x 2048 17.9 and 15.0; 22016 x 2048 27 and 19.7 (k_gemm_w's
+// 64 x 16).
 int choose(uint32_t n, uint32_t m) {
   auto tiles = [&](uint32_t tw, uint32_t mt) { return (n + tw - 1) / tw * ((m + mt - 1) / mt); };
   const bool few = n < 4096;
