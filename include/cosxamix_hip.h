@@ -33,8 +33,9 @@
  *     ends with work still queued and another thread takes its scratch; the
  *     host is not blocked, and a growing scratch is reallocated in stream
  *     order. cx_attention's larger calls are ordered among themselves in the
- *     same way, by a buffer that no other call uses. Under stream capture the scratch cannot grow (CX_EINVAL: make
- *     the call once before capturing) and the caller orders the graph's
+ *     same way, by a buffer that no other call uses. Under stream capture the
+ *     scratch cannot grow (CX_EINVAL: make the call once before capturing) and
+ *     the caller orders the graph's
  *     launches. A cx_model and its caches are used by one thread at a time;
  *     the reference serialises generation behind a Mutex
  *     (src/engine_own.rs:62,185).
