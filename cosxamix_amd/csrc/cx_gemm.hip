@@ -1208,12 +1208,16 @@ Config config(int id, gemm_kernel* k) {
 // Weights in registers (k_gemm_w) where its tiles give the chip enough
 // workgroups, the larger tile first. Whole calls (the quantization with it), us,
 // Q4_K, beside the best of k_gemm's tiles:
-//   64 x 64: 11008 x 2048 m = 512 73, 103, m = 256 45, 59; 4096 x 4096 m = 512 58, 75
+//   64 x 64: 11008 x 2048 m = 512 73, 103, m = 256 45, 59; 4096 x 4096 m = 512 58, 75.
+//     Not for m <= 32, half of it padding: 151936 x 2048 m = 32 103, in 64 x 32 74
 //   64 x 32: 11008 x 2048 m = 128 31, 36; 4096 x 4096 m = 256 39, 42; 2048 x 11008
 //     m = 512 88, 96 (its 512 workgroups; at m = 256 76, 66: k_gemm)
 //   64 x 16: no better than k_gemm's 64 x 16 and 64 x 32, and no worse than by 10%:
 //     4096 x 4096 m = 64 26.5, 26.3, m = 128 29.9, 30.2; 4096 x 14336 (Q5_K) m = 64
-//     78, 71; 2048 x 11008 m = 128 57, 54, 1847 x 2048 m = 389 33, 26: k_gemm
+//     78, 71; 2048 x 11008 m = 128 57, 54, 1847 x 2048 m = 389 33, 26: k_gemm. Not
+//     past two rounds of workgroups: 9000 x 4096 m = 64 40 (Q5_K 47), in 64 x 32 37
+//     (40), 16500 x 2048 m = 32 25.6 (29.1), 23.2 (24.6); nor, for m <= 32, past one:
+//     11008 x 2048 m = 32 19.6 (Q5_K 22.2), in k_gemm's 64 x 32 19.6 (20.8)
 // Otherwise, with m <= 16 rows of many weights, 64 x 16 of k_gemm (11008 x 2048 17.9;
 // 16 x 16 20.8), and for few weight rows (n < 4096: 2048 x 11008 and the q/o/k/v
 // shapes) the largest k_gemm tile (64 x 64, 64 x 32, then 32 x 32) that gives at
@@ -1230,9 +1234,11 @@ int choose(uint32_t n, uint32_t m) {
   auto tiles = [&](uint32_t tw, uint32_t mt) { return (n + tw - 1) / tw * ((m + mt - 1) / mt); };
   const bool few = n < 4096;
   if (m > 16) {
-    if (tiles(64, 64) >= (few ? 768u : 440u)) return 8;
+    if (m > 32 && tiles(64, 64) >= (few ? 768u : 440u)) return 8;
     if (tiles(64, 32) >= (few ? 512u : 300u)) return 7;
-    if (!few && tiles(64, 16) >= 128) return 6;
+    const uint32_t t16 = tiles(64, 16);
+    if (!few && t16 >= (m <= 32 ? 513u : 528u)) return 7;
+    if (!few && t16 >= 128) return m <= 32 && t16 >= 264 ? 3 : 6;
   } else if (!few) {
     return 2;
   }

@@ -54,6 +54,8 @@ def check(dev, t, n, k, m, wild=False, shift=0):
 @pytest.mark.parametrize("t", REG, ids=str)
 @pytest.mark.parametrize("n,k,m", [
     (4096, 256, 17), (4097, 512, 33), (4159, 768, 129),   # 64 x 16
+    (8449, 256, 29), (9001, 512, 32),  # up to 32 rows past one round of those: k_gemm's 64 x 32
+    (8449, 512, 61), (16400, 256, 19), (28225, 256, 32),  # past two, or 64 rows half empty: 64 x 32
     (4096, 256, 131), (4161, 512, 161), (4223, 768, 255),  # 64 x 32
     (4096, 256, 433), (4097, 768, 449), (10001, 512, 193),  # 64 x 64
     (2048, 256, 511), (2111, 512, 500), (3073, 256, 963)])  # few weight rows
